@@ -187,7 +187,7 @@ __device__ inline void coarse_block_sum(double* acc, double (*sh)[N])
 }
 
 // r_c = P^T r: one workgroup per aggregate over its vertex list
-__global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_restrict(int K, const int* __restrict__ aptr,
+__global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_restrict(int K, int nfree, const int* __restrict__ aptr,
                                                                   const int* __restrict__ avert,
                                                                   const double* __restrict__ Ps,
                                                                   const double* __restrict__ r,
@@ -200,7 +200,9 @@ __global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_restrict(int K, const i
     double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     for (int j = aptr[a] + (int)threadIdx.x; j < aptr[a + 1]; j += COARSE_BLOCK) {
         const int v = avert[j];
-        const double* Pv = Ps + 18 * (size_t)j;
+        double Pv[18];
+#pragma unroll
+        for (int m = 0; m < 18; ++m) Pv[m] = Ps[(size_t)m * nfree + j];
         const double r0 = r[3 * v], r1 = r[3 * v + 1], r2 = r[3 * v + 2];
 #pragma unroll
         for (int m = 0; m < 6; ++m) acc[m] += Pv[m] * r0 + Pv[6 + m] * r1 + Pv[12 + m] * r2;
@@ -216,7 +218,7 @@ __global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_restrict(int K, const i
 
 // one workgroup per aggregate a: e = rows 6a..6a+5 of A_c^-1 times r_c, the
 // partial r_c . e_c of those rows, and z += P_v e for the vertices of a
-__global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_solve(int K, int ncd, const int* __restrict__ aptr,
+__global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_solve(int K, int ncd, int nfree, const int* __restrict__ aptr,
                                                                const int* __restrict__ avert,
                                                                const double* __restrict__ Ps,
                                                                const double* __restrict__ Ainv,
@@ -260,7 +262,9 @@ __global__ void __launch_bounds__(COARSE_BLOCK) k_coarse_solve(int K, int ncd, c
     }
     for (int j = aptr[a] + (int)threadIdx.x; j < aptr[a + 1]; j += COARSE_BLOCK) {
         const int v = avert[j];
-        const double* Pv = Ps + 18 * (size_t)j;
+        double Pv[18];
+#pragma unroll
+        for (int m = 0; m < 18; ++m) Pv[m] = Ps[(size_t)m * nfree + j];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             double s = 0.0;
@@ -426,6 +430,7 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
     const int ncd = 6 * K;
     C.K = K;
     C.ncd = ncd;
+    C.nfree = nfree;
     int* d_agg = C.agg.upload_get(agg.data(), nV, s);
     C.aptr.upload(aptr.data(), aptr.size(), s);
     C.avert.upload(avert.data(), avert.size(), s);
@@ -434,7 +439,7 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
         // the apply kernels read P by slot, so its loads do not wait for avert's
         std::vector<double> Ps(18 * (size_t)nfree);
         for (int j = 0; j < nfree; ++j)
-            for (int q = 0; q < 18; ++q) Ps[18 * (size_t)j + q] = P[18 * (size_t)avert[j] + q];
+            for (int q = 0; q < 18; ++q) Ps[(size_t)q * nfree + j] = P[18 * (size_t)avert[j] + q];
         C.Ps.upload(Ps.data(), Ps.size(), s);
     }
     // A_c = P^T A P, summed per aggregate pair in block order
@@ -495,8 +500,8 @@ void coarse_apply(LinWork& L, hipStream_t s, int nV, const double* r, double* z,
 {
     (void)nV;
     CoarseWork& C = L.coarse;
-    IDP_LAUNCH(k_coarse_restrict, C.K, COARSE_BLOCK, 0, s, C.K, C.aptr.p, C.avert.p, C.Ps.p, r, flag, C.rc.p);
-    IDP_LAUNCH(k_coarse_solve, C.K, COARSE_BLOCK, 0, s, C.K, C.ncd, C.aptr.p, C.avert.p, C.Ps.p, C.Ainv.p, C.rc.p,
+    IDP_LAUNCH(k_coarse_restrict, C.K, COARSE_BLOCK, 0, s, C.K, C.nfree, C.aptr.p, C.avert.p, C.Ps.p, r, flag, C.rc.p);
+    IDP_LAUNCH(k_coarse_solve, C.K, COARSE_BLOCK, 0, s, C.K, C.ncd, C.nfree, C.aptr.p, C.avert.p, C.Ps.p, C.Ainv.p, C.rc.p,
                flag, C.part.p + (size_t)parity * C.nsb, z);
 }
 

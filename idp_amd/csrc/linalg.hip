@@ -540,10 +540,8 @@ __device__ inline void cl_apply(int4 cm, const double* __restrict__ Z, int nV, i
 
 // ---------------------------------------------------------------------------
 // Block-Jacobi PCG as two kernels per iteration, enqueued in chunks with no
-// host synchronisation inside a chunk.  A grid-wide barrier inside one
-// persistent kernel costs a device-scope release/acquire per block (the
-// eight XCD L2s are not coherent for ordinary device memory), which grows
-// with the block count; a kernel boundary does that once.
+// host synchronisation inside a chunk (smaller systems run as one kernel,
+// k_pcg_team below).
 //  * k_pcg_spmv(it): every block re-reduces the previous update's partials
 //    (r.z, r.r) in a fixed order, decides convergence identically, forms
 //    p_it = z + beta p_(it-1) on the fly and computes q = A p_it with a group
@@ -830,6 +828,7 @@ __global__ void __launch_bounds__(PCG_UPD_BLOCK) k_pcg_init(PcgArgs A)
             A.x[3 * v + i] = w ? gamma * A.x[3 * v + i] : 0.0;
             A.r[3 * v + i] = rv[i];
             A.z[3 * v + i] = zv[i];
+            A.pbuf[3 * ((size_t)A.nV + v) + i] = 0.0;  // p before the first iteration
             drz += rv[i] * zv[i];
             drr += rv[i] * rv[i];
             dbb += bi * bi;
@@ -1150,6 +1149,758 @@ __global__ void __launch_bounds__(PCG_UPD_BLOCK * PCG_UPD_WAVES_MAX) k_pcg_updat
     }
 }
 
+// ---------------------------------------------------------------------------
+// A whole PCG solve as one kernel.  Each instance's solve is run by a team of
+// workgroups that are resident together (or by one); they meet where the two
+// kernels above would end, and nothing is launched or read back until the
+// solve stops.  Same sums in the same order as those kernels (and
+// k_coarse_restrict / k_coarse_solve), so the results are the same bit for
+// bit, whatever the team size.
+//
+// Vectors that other workgroups of the team read (z, p, q, r) go through
+// agent-scope relaxed atomic accesses: they reach the memory the eight XCDs
+// share without the write-back and invalidation of a whole L2 that a release
+// / acquire fence costs, so the matrix, the preconditioner and A_c^-1, read
+// with plain loads, stay in each XCD's L2 (or in registers, for the first
+// rows of a workgroup) over the iterations.  The workgroups meet on the
+// partial sums themselves: a partial is published as two 64-bit words, half
+// of its bits and the iteration's tag in each, after every wavefront's vector
+// stores were acknowledged, and a reader polls until both tags match.  A
+// team of one workgroup (ONE) uses plain accesses and LDS.
+// ---------------------------------------------------------------------------
+constexpr int TEAM_THREADS = 512;  // 2 wavefronts per SIMD: 256 registers a lane, room for the first rows' blocks
+constexpr int TEAM_WAVES = TEAM_THREADS / 64;
+constexpr int TEAM_MAX = 256;      // workgroups of a launch at most: one per CU
+constexpr int TEAM_ROWS = 128;     // rows of a workgroup: two per 8 lanes in the SpMV, 4 lanes a row in the update
+constexpr int TEAM_TASKS = 512;    // coarse aggregates at most (and, fewer, wavefront row sums)
+constexpr int TEAM_VALUES = 1952;  // values of one meeting at most (r_c of 320 aggregates)
+
+struct TeamArgs {
+    const int4* tab;  // per workgroup {instance, rank, team size, 0}; null: one instance, the whole grid
+    const int* vbeg;  // instance vertex ranges (B + 1)
+    const int* it0;   // per instance: iterations of earlier calls (null: 0)
+    // published partials, two words each: p.q (nbA), r.z, r.r and the hand-over mark (2 nbB + B), r_c, r_c . e_c
+    unsigned long long *w_pq, *w_r, *w_rc, *w_cp;
+    unsigned tag0;    // tags of this launch are tag0 + 1 + iteration; larger than any before
+    int* ctl;         // [0] a wait ran out (the launch is void), [1] solves stopped, [2] hand-over after this many
+                      // iterations (0: not yet)
+    int* done;        // per instance: iterations done by this call when handed over
+    int nstart;       // hand-over: solves at launch (0: never)
+    long spin_limit;  // polls of one wait at most
+    // coarse level (one instance; K = 0: none)
+    int K, ncd, nfree;
+    const int *aptr, *avert;
+    const double *Ps, *Ainv;
+};
+
+template <bool ONE, class T>
+__device__ inline T team_ld(const T* p)
+{
+    if (ONE) return *p;
+    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool ONE, class T>
+__device__ inline void team_st(T* p, T v)
+{
+    if (ONE) *p = v;
+    else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+typedef unsigned team_u2 __attribute__((ext_vector_type(2)));
+typedef unsigned team_u4 __attribute__((ext_vector_type(4)));
+
+__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// ends a phase that stored vectors: every wavefront's stores have reached the
+// memory they are read from, then the workgroup's LDS is in step
+__device__ inline void team_stores_done()
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
+__device__ inline __amdgpu_buffer_rsrc_t team_words(const unsigned long long* w, int n)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned long long*>(w), 0, 16 * n, 0x00027000);
+}
+
+// value i of a meeting of n: published (the two words in one store), or (one workgroup) put where team_meet would
+template <bool ONE>
+__device__ inline void team_put(unsigned long long* w, int n, double* val, int i, double v, unsigned tag)
+{
+    if (ONE) {
+        val[i] = v;
+    } else {
+        const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+        const team_u4 d = {(unsigned)b, tag, (unsigned)(b >> 32), tag};
+        __builtin_amdgcn_raw_buffer_store_b128(d, team_words(w, n), 16 * i, 0, 16);
+    }
+}
+
+// waits for the n values of a meeting and leaves them in val (LDS); false
+// when the wait ran out, which voids the launch: every workgroup then leaves
+template <bool ONE>
+__device__ inline bool team_meet(const TeamArgs& T, const unsigned long long* w, int n, unsigned tag, double* val,
+                                 int* bad)
+{
+    if (!ONE) {
+        const __amdgpu_buffer_rsrc_t rs = team_words(w, n);
+        constexpr int M = 4;  // values of a thread whose loads are in flight together
+        for (int base = 0; base < n; base += M * TEAM_THREADS) {
+            team_u4 v[M];
+            bool ok = false;
+            for (long k = 0; k < T.spin_limit && !ok; ++k) {
+                asm volatile("" ::: "memory");  // the loads are made anew in every round
+                ok = true;
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    const int i = base + (int)threadIdx.x + TEAM_THREADS * m;
+                    if (i < n) v[m] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * i, 0, 16);
+                }
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+                    if (base + (int)threadIdx.x + TEAM_THREADS * m < n) ok = ok && v[m][1] == tag && v[m][3] == tag;
+            }
+            if (!ok) {
+                *bad = 1;
+                team_st<false>(T.ctl, 1);
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int i = base + (int)threadIdx.x + TEAM_THREADS * m;
+                if (i < n) val[i] = __longlong_as_double((long long)(((unsigned long long)v[m][2] << 32) | v[m][0]));
+            }
+        }
+    }
+    __syncthreads();
+    return ONE || *bad == 0;
+}
+
+// cross-lane moves of a double within a row of 16 lanes (DPP; an LDS
+// permute has several times the latency, and these sums are serial)
+template <int CTRL, int BANKS>
+__device__ inline double dpp_f64(double old, double x)
+{
+    const long long xi = __double_as_longlong(x), oi = __double_as_longlong(old);
+    const int lo = __builtin_amdgcn_update_dpp((int)oi, (int)xi, CTRL, 0xf, BANKS, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(oi >> 32), (int)(xi >> 32), CTRL, 0xf, BANKS, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline double dpp_xor1(double x) { return dpp_f64<0xB1, 0xf>(0.0, x); }  // quad_perm 1 0 3 2
+__device__ inline double dpp_xor2(double x) { return dpp_f64<0x4E, 0xf>(0.0, x); }  // quad_perm 2 3 0 1
+__device__ inline double dpp_xor4(double x) { return dpp_f64<0x124, 0xA>(dpp_f64<0x12C, 0x5>(0.0, x), x); }  // row_ror
+__device__ inline double dpp_xor8(double x) { return dpp_f64<0x128, 0xf>(0.0, x); }                          // row_ror:8
+
+// wave_sum with the same partners in the same order (240 clocks instead of 600)
+__device__ inline double wave_sum_dpp(double x)
+{
+    {
+        const long long i = __double_as_longlong(x);
+        const auto a = __builtin_amdgcn_permlane32_swap((unsigned)i, (unsigned)i, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap((unsigned)(i >> 32), (unsigned)(i >> 32), false, false);
+        x = __longlong_as_double(((long long)b[0] << 32) | a[0]) + __longlong_as_double(((long long)b[1] << 32) | a[1]);
+    }
+    {
+        const long long i = __double_as_longlong(x);
+        const auto a = __builtin_amdgcn_permlane16_swap((unsigned)i, (unsigned)i, false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap((unsigned)(i >> 32), (unsigned)(i >> 32), false, false);
+        x = __longlong_as_double(((long long)b[0] << 32) | a[0]) + __longlong_as_double(((long long)b[1] << 32) | a[1]);
+    }
+    x += dpp_xor8(x);
+    x += dpp_xor4(x);
+    x += dpp_xor2(x);
+    x += dpp_xor1(x);
+    return x;
+}
+
+// r.z of update block b in the second meeting's values (r.r two further): the
+// two blocks of a chunk fill a 64-byte line, which one workgroup writes
+__device__ inline int team_rblk(int b) { return 4 * (b >> 1) + (b & 1); }
+struct TeamRblk {
+    __device__ int operator()(int b) const { return team_rblk(b); }
+};
+
+// the order of wave_sum_partials over n values (LDS or global memory)
+struct TeamIdent {
+    __device__ int operator()(int i) const { return i; }
+};
+template <class F = TeamIdent>
+__device__ inline double team_sum(const double* part, int n, F at = F())
+{
+    const int lane = threadIdx.x & 63;
+    double acc = 0.0;
+    for (int base = 0; base < n; base += 64 * 8) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int i = base + lane + 64 * k;
+            v[k] = i < n ? part[at(i)] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc += v[k];
+    }
+    return wave_sum_dpp(acc);
+}
+
+// A vector as a buffer resource: its gathers take a 32-bit byte offset (one
+// register of address instead of two per load) and two loads per 3-vector.
+// Cache policy 16 is sc1, the agent-scope access of team_ld.
+struct TeamBuf {
+    __amdgpu_buffer_rsrc_t rs;
+    __device__ TeamBuf(double* p, long n) : rs(__builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(unsigned)(8 * n), 0x00027000)) {}
+    template <bool ONE>
+    __device__ void ld3(unsigned off, unsigned base, double* o) const
+    {
+        const team_u4 a = __builtin_amdgcn_raw_buffer_load_b128(rs, off, base, ONE ? 0 : 16);
+        const team_u2 b = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 16u, base, ONE ? 0 : 16);
+        o[0] = __longlong_as_double((long long)(((unsigned long long)a[1] << 32) | a[0]));
+        o[1] = __longlong_as_double((long long)(((unsigned long long)a[3] << 32) | a[2]));
+        o[2] = __longlong_as_double((long long)(((unsigned long long)b[1] << 32) | b[0]));
+    }
+    template <bool ONE>
+    __device__ double ld1(unsigned off, unsigned base) const
+    {
+        const team_u2 b = __builtin_amdgcn_raw_buffer_load_b64(rs, off, base, ONE ? 0 : 16);
+        return __longlong_as_double((long long)(((unsigned long long)b[1] << 32) | b[0]));
+    }
+};
+
+// one BSR block of a row: slot j of its elastic blocks followed by its
+// contact blocks, and its column.  A slot past the row's end is a zero block
+// on the row itself (no branch; it adds 0).
+struct TeamSlot {
+    int col;
+    double b[9];
+    __device__ void load(const PcgArgs& A, int v, int j, int e0, int ne, int c0, int nc)
+    {
+        col = v;
+#pragma unroll
+        for (int e = 0; e < 9; ++e) b[e] = 0.0;
+        if (j >= ne + nc) return;
+        const bool el = j < ne;
+        const double* __restrict__ val = el ? A.eval : A.cval;
+        const long ld = el ? A.eld : A.cld;
+        const int k = el ? e0 + j : c0 + (j - ne);
+        col = el ? A.ecol[k] : A.ccol[k];
+#pragma unroll
+        for (int e = 0; e < 9; ++e) b[e] = val[e * ld + k];
+    }
+};
+
+// The columns of a workgroup's rows, each once: a set over the instance's
+// vertices (one bit each, with the number of members before each word) and
+// its members in order.  Every iteration reads z and p_old of the first
+// TEAM_COLS members into LDS once, instead of once per block that uses them:
+// a lane's gather of a 24-byte record occupies the CU's address unit for a
+// whole cache line, and 128 rows of about 14 blocks have some 500 columns
+// (row phase of the 64x16x16 bar: 4.2 us with one gather per block).
+constexpr int TEAM_COLS = 1024;
+constexpr int TEAM_SET = TEAM_MAX * TEAM_ROWS / 32;  // words of a set
+struct TeamCols {
+    unsigned* bits;
+    int* before;
+    int* list;
+    double *z, *p;  // 3 per member
+    __device__ int find(int c) const
+    {
+        const unsigned w = bits[c >> 5];
+        return before[c >> 5] + __popc(w & ((1u << (c & 31)) - 1u));
+    }
+};
+
+struct TeamVec {
+    double z[3], p[3];
+    // z and p_old (byte po of the p buffer) at column col, member k of the set
+    template <bool ONE>
+    __device__ void load(const TeamBuf& bz, const TeamBuf& bp, unsigned po, const TeamCols& C, int k, int col)
+    {
+        if (k < TEAM_COLS) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                z[d] = C.z[3 * k + d];
+                p[d] = C.p[3 * k + d];
+            }
+        } else {
+            bz.ld3<ONE>(24u * (unsigned)col, 0, z);
+            bp.ld3<ONE>(24u * (unsigned)col, po, p);
+        }
+    }
+    // y += B z, w += B p (row_spmv's sums)
+    __device__ void add(const TeamSlot& S, double* y, double* w) const
+    {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) y[i] += S.b[3 * i] * z[0] + S.b[3 * i + 1] * z[1] + S.b[3 * i + 2] * z[2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) w[i] += S.b[3 * i] * p[0] + S.b[3 * i + 1] * p[1] + S.b[3 * i + 2] * p[2];
+    }
+};
+
+// what a lane of the update keeps of its row: lane b of a row's four holds
+// the row's preconditioner block for cluster member b and that member's
+// residual (every holder of a residual updates it alike); the lane of the row
+// itself also holds x
+struct TeamRow {
+    int v, u;  // row, member (-1: none)
+    bool own, single;
+    double Z[9], r[3], x[3];
+    template <bool ONE>
+    __device__ void load(const PcgArgs& A, int row, int vend, int b, const double* r_in)
+    {
+        v = row;
+        u = -1;
+        own = single = false;
+#pragma unroll
+        for (int e = 0; e < 9; ++e) Z[e] = 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) r[d] = x[d] = 0.0;
+        if (v >= vend) return;
+        const int4 cm = A.cm4[v];
+        single = cm.y < 0;
+        u = b == 0 ? cm.x : b == 1 ? cm.y : b == 2 ? cm.z : cm.w;
+        if (single && b == 0) u = v;
+        if (u < 0) return;
+        own = u == v;
+        const double* o = A.Z + 9 * ((size_t)b * A.nV + v);
+#pragma unroll
+        for (int e = 0; e < 9; ++e) Z[e] = o[e];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            r[d] = team_ld<ONE>(r_in + 3 * (size_t)u + d);
+            if (own) x[d] = A.x[3 * (size_t)v + d];
+        }
+    }
+};
+
+// a row's block count and its first two slots of this lane (rows past the end: zero blocks on row v0)
+struct TeamTask {
+    int n, ka, kb, ko;  // blocks of the row; members of the column set of the two slots and of the row
+    TeamSlot a, b;
+    __device__ void load(const PcgArgs& A, int v, int vend, int v0, int gl)
+    {
+        int e0 = 0, ne = 0, c0 = 0, nc = 0;
+        if (v < vend) row_extents(A, v, e0, ne, c0, nc);
+        else v = v0;
+        n = ne + nc;
+        a.load(A, v, gl, e0, ne, c0, nc);
+        b.load(A, v, gl + 8, e0, ne, c0, nc);
+    }
+};
+
+// p and q = A p of row v (8 lanes, row_spmv's order); the wavefront's sum of p.q
+template <bool ONE>
+__device__ inline double team_row(const PcgArgs& A, const TeamBuf& bz, const TeamBuf& bp, unsigned po, const TeamCols& C,
+                                  const TeamTask& K, int v, int vend, int v0, int gl, double beta, double* pn)
+{
+    double y[3] = {0.0, 0.0, 0.0}, w[3] = {0.0, 0.0, 0.0};
+    double zo, poo;  // this lane's component of the row's own z and p_old
+    {
+        TeamVec Va, Vb;
+        Va.load<ONE>(bz, bp, po, C, K.ka, K.a.col);
+        Vb.load<ONE>(bz, bp, po, C, K.kb, K.b.col);
+        const int g = min(gl, 2);
+        if (K.ko < TEAM_COLS) {
+            zo = C.z[3 * K.ko + g];
+            poo = C.p[3 * K.ko + g];
+        } else {
+            const unsigned i = 24u * (unsigned)(v < vend ? v : v0) + 8u * (unsigned)g;
+            zo = bz.ld1<ONE>(i, 0);
+            poo = bp.ld1<ONE>(i, po);
+        }
+        Va.add(K.a, y, w);
+        Vb.add(K.b, y, w);
+    }
+    if (K.n > 16) {  // longer rows: the rest of their blocks from memory
+        int e0, ne, c0, nc;
+        row_extents(A, v, e0, ne, c0, nc);
+        for (int j = gl + 16; j < K.n; j += 8) {
+            TeamSlot S;
+            TeamVec u;
+            S.load(A, v, j, e0, ne, c0, nc);
+            u.load<ONE>(bz, bp, po, C, C.find(S.col - v0), S.col);
+            u.add(S, y, w);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] += beta * w[i];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] += dpp_xor4(y[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] += dpp_xor2(y[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) y[i] += dpp_xor1(y[i]);
+    double yl = y[2];
+    yl = gl == 1 ? y[1] : yl;
+    yl = gl == 0 ? y[0] : yl;
+    double d = 0.0;
+    if (gl < 3 && v < vend) {
+        const size_t i = 3 * (size_t)v + gl;
+        const double pv = zo + beta * poo;
+        team_st<ONE>(pn + i, pv);
+        team_st<ONE>(A.q + i, yl);
+        d = pv * yl;
+    }
+    return wave_sum_dpp(d);
+}
+
+// COARSE: with the coarse level (T.K > 0)
+template <bool ONE, bool COARSE>
+__global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T)
+{
+    __shared__ double wt[TEAM_TASKS];
+    __shared__ double val[TEAM_VALUES];
+    __shared__ double rowz[TEAM_ROWS], rowr[TEAM_ROWS];
+    __shared__ unsigned cbits[TEAM_SET];
+    __shared__ int cbefore[TEAM_SET], clist[TEAM_COLS];
+    __shared__ double cz[3 * TEAM_COLS], cp[3 * TEAM_COLS];
+    const TeamCols C{cbits, cbefore, clist, cz, cp};
+    __shared__ double sh[8];
+    __shared__ double shc[TEAM_WAVES][6];
+    __shared__ int bad, cwave[TEAM_WAVES];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int inst = 0, rank = blockIdx.x, size = gridDim.x;
+    if (T.tab) {
+        const int4 t = T.tab[blockIdx.x];
+        inst = uni(t.x);
+        rank = uni(t.y);
+        size = uni(t.z);
+    }
+    if (A.flag[inst] != 0) return;  // not solving (uniform over the team: written at a solve's end only)
+    const int v0 = uni(T.vbeg[inst]), v1 = uni(T.vbeg[inst + 1]);
+    const int pb = uni(A.bpbeg[inst]), nb = uni(A.bpbeg[inst + 1]) - pb;
+    const int ab = uni(A.apbeg[inst]), na = uni(A.apbeg[inst + 1]) - ab;
+    // this workgroup's 64-row update blocks and the 32-row SpMV blocks of the same rows
+    const int b0 = (int)((long)nb * rank / size), b1 = (int)((long)nb * (rank + 1) / size);
+    const int u0 = 2 * b0, nu = min(2 * b1, na) - u0;
+    const int rb = v0 + 64 * b0, re = min(v0 + 64 * b1, v1);
+    const int it_first = T.it0 ? uni(T.it0[inst]) : 0;
+    const TeamBuf bz(A.z, 3L * A.nV), bp(A.pbuf, 6L * A.nV), bq(A.q, 3L * A.nV), br(A.r, 6L * A.nV);
+    unsigned long long* w_pq = T.w_pq + 2 * (size_t)ab;
+    const int nr = 4 * ((nb + 1) / 2) + 1;  // values of the second meeting; the last: the hand-over mark
+    unsigned long long* w_r = T.w_r + 2 * (2 * (size_t)pb + 8 * inst);
+    double* sci = A.scal + 3 * inst;
+    double rz = 0.0, rr = 0.0, rzo = 1.0, bb = 0.0;
+    int hand = 0;
+    if (tid == 0) bad = 0;
+    // ---- the workgroup's blocks and update state stay in registers
+    const int gl = lane & 7;
+    const int row0 = rb + 8 * wave + (lane >> 3);  // SpMV rows: row0 and row0 + 64
+    TeamTask K0, K1;
+    K0.load(A, row0, re, v0, gl);
+    K1.load(A, row0 + 64, re, v0, gl);
+    int ncol = 0;
+    {
+        const int nw = (v1 - v0 + 31) >> 5;
+        for (int i = tid; i < nw; i += TEAM_THREADS) cbits[i] = 0u;
+        __syncthreads();
+        auto mark = [&](int col) { atomicOr(&cbits[(col - v0) >> 5], 1u << ((col - v0) & 31)); };
+        for (int k = 0; k < 2; ++k) {
+            const int v = row0 + 64 * k;
+            if (v >= re) continue;
+            int e0, ne, c0, nc;
+            row_extents(A, v, e0, ne, c0, nc);
+            for (int j = gl; j < ne + nc; j += 8) mark(j < ne ? A.ecol[e0 + j] : A.ccol[c0 + j - ne]);
+        }
+        if (tid == 0) mark(v0);  // where the lanes past the rows' end point
+        __syncthreads();
+        // members before each word: a run of words per thread, then the runs' sums
+        const int per = (nw + TEAM_THREADS - 1) / TEAM_THREADS;
+        const int w0 = min(tid * per, nw), w1 = min(w0 + per, nw);
+        int cnt = 0;
+        for (int i = w0; i < w1; ++i) cnt += __popc(cbits[i]);
+        int inc = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += t;
+        }
+        if (lane == 63) cwave[wave] = inc;
+        __syncthreads();
+        int at = inc - cnt;
+        for (int w = 0; w < TEAM_WAVES; ++w) {
+            if (w < wave) at += cwave[w];
+            ncol += cwave[w];
+        }
+        for (int i = w0; i < w1; ++i) {
+            cbefore[i] = at;
+            for (unsigned b = cbits[i]; b; b &= b - 1u) {
+                if (at < TEAM_COLS) clist[at] = v0 + 32 * i + __ffs((int)b) - 1;
+                ++at;
+            }
+        }
+        __syncthreads();
+        ncol = min(uni(ncol), TEAM_COLS);
+        K0.ka = C.find(K0.a.col - v0);
+        K0.kb = C.find(K0.b.col - v0);
+        K1.ka = C.find(K1.a.col - v0);
+        K1.kb = C.find(K1.b.col - v0);
+        K0.ko = C.find((row0 < re ? row0 : v0) - v0);
+        K1.ko = C.find((row0 + 64 < re ? row0 + 64 : v0) - v0);
+    }
+    const int ur = 16 * wave + (lane >> 2), ub = lane & 3;  // update: row, cluster member
+    TeamRow R0;
+    R0.load<true>(A, rb + ur, re, ub, A.r + (size_t)(it_first & 1) * 3 * A.nV);
+    // ---- the sums that the launch starts from
+    {
+        const int par = it_first & 1;
+        double s = 0.0;
+        if (wave == 0) s = team_sum(A.part_rz + par * A.nbB + pb, nb);
+        else if (wave == 1) s = team_sum(A.part_rr + par * A.nbB + pb, nb);
+        else if (wave == 2 && COARSE) s = team_sum(A.cpart + par * T.K, T.K);
+        else if (wave == 3) s = team_sum(it_first > 0 ? A.part_rz + (par ^ 1) * A.nbB + pb : A.part_rr + A.nbB + pb, nb);
+        if (wave < 4 && lane == 0) sh[wave] = s;
+        __syncthreads();
+        rz = sh[0];
+        rr = sh[1];
+        if (COARSE) rz += sh[2];
+        if (it_first > 0) {
+            rzo = sh[3];
+            bb = sci[0];
+        } else {
+            bb = sh[3];
+        }
+    }
+    int state = 0;  // 1 converged, 4 iteration limit, 2 breakdown, -1 handed over
+    int it = it_first;
+    for (;; ++it) {
+        const unsigned tag = T.tag0 + 1u + (unsigned)(it - it_first);
+        const int par = it & 1;
+        // the same decisions in every workgroup of the team
+        if (!(bb > 0.0) || (it > 0 && rr <= A.rtol2 * bb)) {
+            state = 1;
+            break;
+        }
+        if (it >= A.maxit) {
+            state = 4;
+            break;
+        }
+        if (hand) {
+            state = -1;
+            break;
+        }
+        const double beta = it > 0 ? rz / rzo : 0.0;
+        rzo = rz;
+        // ---- p = z + beta p_old, q = A p and the partials of p.q
+        const unsigned po = (unsigned)(par ^ 1) * 24u * (unsigned)A.nV;  // p_old is zero at iteration 0
+        const unsigned pc = (unsigned)par * 24u * (unsigned)A.nV;
+        double* pn = A.pbuf + (size_t)par * 3 * A.nV;
+        for (int i = tid; i < ncol; i += TEAM_THREADS) {
+            const unsigned off = 24u * (unsigned)clist[i];
+            bz.ld3<ONE>(off, 0, cz + 3 * i);
+            bp.ld3<ONE>(off, po, cp + 3 * i);
+        }
+        __syncthreads();
+        {
+            const double da = team_row<ONE>(A, bz, bp, po, C, K0, row0, re, v0, gl, beta, pn);
+            const double db = team_row<ONE>(A, bz, bp, po, C, K1, row0 + 64, re, v0, gl, beta, pn);
+            if (lane == 0) {
+                wt[wave] = da;
+                wt[8 + wave] = db;
+            }
+        }
+        team_stores_done();
+        if (tid < nu) {
+            double a = 0.0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) a += wt[4 * tid + k];
+            team_put<ONE>(w_pq, na, val, u0 + tid, a, tag);
+        }
+        if (!team_meet<ONE>(T, w_pq, na, tag, val, &bad)) return;
+        // ---- alpha, x, r, z = M r and the partials of r.z, r.r
+        double* r_out = A.r + (size_t)(par ^ 1) * 3 * A.nV;
+        double q[3] = {0.0, 0.0, 0.0}, pv[3] = {0.0, 0.0, 0.0};
+        if (R0.u >= 0) {
+            bq.ld3<ONE>(24u * (unsigned)R0.u, 0, q);
+            if (R0.own) bp.ld3<ONE>(24u * (unsigned)R0.u, pc, pv);
+        }
+        if (wave == 0) {
+            const double s = team_sum(val, na);
+            if (lane == 0) sh[4] = s;
+        }
+        __syncthreads();
+        const double pq = sh[4];
+        if (!(pq > 0.0)) {
+            state = 2;
+            break;
+        }
+        const double alpha = rz / pq;
+        {
+            double t[3], zv[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) R0.r[d] = R0.r[d] - alpha * q[d];
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                t[d] = R0.Z[3 * d] * R0.r[0] + R0.Z[3 * d + 1] * R0.r[1] + R0.Z[3 * d + 2] * R0.r[2];
+            // the members' terms in order (every lane of the row gets the sum)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const double t0 = dpp_f64<0x00, 0xf>(0.0, t[d]), t1 = dpp_f64<0x55, 0xf>(0.0, t[d]),
+                             t2 = dpp_f64<0xAA, 0xf>(0.0, t[d]), t3 = dpp_f64<0xFF, 0xf>(0.0, t[d]);
+                zv[d] = R0.single ? t0 : ((t0 + t1) + t2) + t3;
+            }
+            if (R0.own) {
+                const size_t i0 = 3 * (size_t)R0.v;
+                double drz = 0.0, drr = 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    R0.x[d] = R0.x[d] + alpha * pv[d];
+                    team_st<ONE>(r_out + i0 + d, R0.r[d]);
+                    team_st<ONE>(A.z + i0 + d, zv[d]);
+                    drz += R0.r[d] * zv[d];
+                    drr += R0.r[d] * R0.r[d];
+                }
+                rowz[ur] = drz;
+                rowr[ur] = drr;
+            } else if (ub == 0 && R0.v >= re) {
+                rowz[ur] = rowr[ur] = 0.0;
+            }
+        }
+        team_stores_done();
+        // the workgroup's (at most) two 64-row blocks; lanes 0..3 publish their r.z and r.r together
+        if (wave == 0) {
+            const double z0 = wave_sum_dpp(rowz[lane]), z1 = wave_sum_dpp(rowz[64 + lane]);
+            const double q0 = wave_sum_dpp(rowr[lane]), q1 = wave_sum_dpp(rowr[64 + lane]);
+            const int blk = b0 + (lane & 1);
+            if (lane < 4 && blk < b1) {
+                const double s = lane < 2 ? (lane ? z1 : z0) : (lane & 1 ? q1 : q0);
+                // for a call that continues this solve
+                (lane < 2 ? A.part_rz : A.part_rr)[(par ^ 1) * A.nbB + pb + blk] = s;
+                team_put<ONE>(w_r, nr, val, team_rblk(blk) + (lane & 2), s, tag);
+            }
+        }
+        // an odd number of blocks: the last line's other half is published too, so that all of it is waited for
+        if (wave == 1 && lane < 2 && (nb & 1) && rank == size - 1)
+            team_put<ONE>(w_r, nr, val, team_rblk(nb) + 2 * lane, 0.0, tag);
+        if (T.nstart && rank == 0 && tid == 0) {
+            // half of the solves have stopped: hand over after as many iterations again
+            const int half = team_ld<false>(T.ctl + 2);
+            team_put<ONE>(w_r, nr, val, nr - 1, half > 0 && it + 1 - it_first >= 2 * half ? 1.0 : 0.0, tag);
+        }
+        if (!team_meet<ONE>(T, w_r, T.nstart ? nr : nr - 1, tag, val, &bad)) return;
+        if (wave == 0) {
+            const double s = team_sum(val, nb, TeamRblk());
+            if (lane == 0) sh[0] = s;
+        } else if (wave == 1) {
+            const double s = team_sum(val + 2, nb, TeamRblk());
+            if (lane == 0) sh[1] = s;
+        } else if (wave == 2 && lane == 0) {
+            sh[5] = T.nstart ? val[nr - 1] : 0.0;
+        }
+        if (COARSE) {
+            __syncthreads();  // val is read above and written by the next meeting
+            // ---- coarse level: r_c = P^T r, then e_c = A_c^-1 r_c and z += P e_c; 256 threads per aggregate
+            const int q4 = tid >> 8, t4 = tid & 255;
+            for (int a0 = rank; a0 < T.K; a0 += 2 * size) {
+                const int a = a0 + q4 * size;
+                double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                if (a < T.K) {
+                    const int j1 = T.aptr[a + 1];
+                    for (int j = T.aptr[a] + t4; j < j1; j += 256) {
+                        double x[3], Pv[18];
+                        br.ld3<ONE>(24u * (unsigned)T.avert[j], (unsigned)(par ^ 1) * 24u * (unsigned)A.nV, x);
+#pragma unroll
+                        for (int m = 0; m < 18; ++m) Pv[m] = T.Ps[(size_t)m * T.nfree + j];
+#pragma unroll
+                        for (int m = 0; m < 6; ++m) acc[m] += Pv[m] * x[0] + Pv[6 + m] * x[1] + Pv[12 + m] * x[2];
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < 6; ++m) {
+                    const double s = wave_sum_dpp(acc[m]);
+                    if (lane == 0) shc[wave][m] = s;
+                }
+                __syncthreads();
+                if (a < T.K && t4 < 6) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) s += shc[4 * q4 + k][t4];
+                    team_put<ONE>(T.w_rc, T.ncd, val, 6 * a + t4, s, tag);
+                }
+                __syncthreads();
+            }
+            if (!team_meet<ONE>(T, T.w_rc, T.ncd, tag, val, &bad)) return;
+            for (int a0 = rank; a0 < T.K; a0 += 2 * size) {
+                const int a = a0 + q4 * size;
+                double e[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                if (a < T.K) {
+                    const double* Ar = T.Ainv + (size_t)(6 * a) * T.ncd;
+#pragma unroll 4
+                    for (int j = t4; j < T.ncd; j += 256) {
+                        const double rj = val[j];
+#pragma unroll
+                        for (int m = 0; m < 6; ++m) e[m] += Ar[(size_t)m * T.ncd + j] * rj;
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < 6; ++m) {
+                    const double s = wave_sum_dpp(e[m]);
+                    if (lane == 0) shc[wave][m] = s;
+                }
+                __syncthreads();
+                if (a < T.K) {
+#pragma unroll
+                    for (int m = 0; m < 6; ++m) {
+                        double s = 0.0;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) s += shc[4 * q4 + k][m];
+                        e[m] = s;
+                    }
+                    if (t4 == 0) {
+                        double d = 0.0;
+#pragma unroll
+                        for (int m = 0; m < 6; ++m) d += val[6 * a + m] * e[m];
+                        wt[a] = d;
+                    }
+                    const int j1 = T.aptr[a + 1];
+                    for (int j = T.aptr[a] + t4; j < j1; j += 256) {
+                        const int v = T.avert[j];
+                        double x[3], Pv[18];
+                        bz.ld3<ONE>(24u * (unsigned)v, 0, x);
+#pragma unroll
+                        for (int m = 0; m < 18; ++m) Pv[m] = T.Ps[(size_t)m * T.nfree + j];
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) {
+                            double s = 0.0;
+#pragma unroll
+                            for (int m = 0; m < 6; ++m) s += Pv[6 * d + m] * e[m];
+                            team_st<ONE>(A.z + 3 * (size_t)v + d, x[d] + s);
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+            team_stores_done();
+            for (int a = rank + tid * size; a < T.K; a += TEAM_THREADS * size) team_put<ONE>(T.w_cp, T.K, val, a, wt[a], tag);
+            if (!team_meet<ONE>(T, T.w_cp, T.K, tag, val, &bad)) return;
+            if (wave == 0) {
+                const double s = team_sum(val, T.K);
+                if (lane == 0) sh[2] = s;
+            }
+        }
+        __syncthreads();
+        rz = sh[0];
+        rr = sh[1];
+        hand = sh[5] != 0.0;
+        if (COARSE) rz += sh[2];
+    }
+    // ---- the solve stopped or is handed over
+    if (R0.own && it > it_first)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) A.x[3 * (size_t)R0.v + d] = R0.x[d];
+    if (rank != 0 || tid != 0) return;
+    if (state != 2) sci[0] = bb;
+    if (state == -1) {  // the state is on the device: a later call continues at this iteration
+        T.done[inst] = it - it_first;
+        return;
+    }
+    A.flag[inst] = state;
+    if (state != 2) sci[1] = rr;
+    sci[2] = (double)it;
+    if (T.nstart) {  // once half of the solves have stopped, the others learn after how many iterations
+        const int n = atomicAdd(T.ctl + 1, 1) + 1;
+        if (2 * n >= T.nstart) atomicCAS(T.ctl + 2, 0, max(1, it - it_first));
+    }
+}
+
 // generic deterministic sum of partials -> out[0]
 __global__ void __launch_bounds__(RB) k_sum_partials(int npart, const double* __restrict__ part,
                                                      double* __restrict__ out)
@@ -1325,13 +2076,97 @@ void init_erow(LinWork& L, hipStream_t s, const MeshDev& m, const std::vector<in
     L.erow.upload(rowof.data(), rowof.size(), s);
 }
 
+__global__ void k_zero_words(long n, unsigned long long* __restrict__ w)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) w[i] = 0ull;
+}
+
+// also clears the team kernel's words (nteam of them)
 __global__ void k_pcg_start(int B, const unsigned char* __restrict__ solve, int* __restrict__ flag,
-                            int* __restrict__ err)
+                            int* __restrict__ err, int nteam, int* __restrict__ team)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nteam) team[i] = 0;
     if (i >= B) return;
     flag[i] = (solve && !solve[i]) ? 3 : 0;  // new and continued solves iterate
     err[i] = 0;
+}
+
+// Runs the solves of the instances in `run` with k_pcg_team; false where the
+// two-kernel loop is used instead:
+//  - more rows than TEAM_MAX workgroups hold (32,768).  With the rest of the
+//    rows read from memory an iteration of 24 cubes (41,580 rows) took 18 us,
+//    against 15 us in the two kernels;
+//  - a coarse level of more than two aggregates per workgroup and 256-thread
+//    half: a thin sheet of 625 free vertices (10 workgroups) has 320 of them,
+//    and took 1.2 ms more per solve than the four kernels.
+// Below, per iteration and with launch gaps: 81 rows 24 -> 5 us, 18,785 rows
+// with 100-130 aggregates 40 -> 30-39 us.
+bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, const std::vector<char>& run, int* team,
+              bool coarse, bool handover)
+{
+    const int B = I.B;
+    std::vector<int4> tab;
+    bool one = true;
+    int nrun = 0;
+    for (int i = 0; i < B; ++i)
+        if (run[i]) {
+            ++nrun;
+            const int nb = I.pcg_upd.h_pbeg[i + 1] - I.pcg_upd.h_pbeg[i];
+            const int t = (nb + 1) / 2;  // TEAM_ROWS rows per workgroup
+            if (tab.size() + t > TEAM_MAX) return false;
+            for (int k = 0; k < t; ++k) tab.push_back(make_int4(i, k, t, 0));
+            one = one && t == 1;
+        }
+    if (nrun == 0) return false;
+    if (coarse && L.coarse.K > 4 * (int)tab.size()) return false;
+    TeamArgs T;
+    T.tab = B == 1 ? nullptr : L.team_tab.upload_get(tab.data(), tab.size(), s);
+    T.vbeg = I.d_vbeg.p;
+    T.it0 = nullptr;
+    for (int i = 0; i < B; ++i)
+        if (run[i] && L.h_it0[i]) T.it0 = L.team_it0.upload_get(L.h_it0.data(), B, s);
+    T.K = coarse ? L.coarse.K : 0;
+    T.ncd = L.coarse.ncd;
+    T.nfree = L.coarse.nfree;
+    if (T.K && (T.ncd > TEAM_VALUES || T.K > TEAM_TASKS)) return false;
+    // published words; tags only grow, so words of earlier launches never match (cleared when they would wrap)
+    const size_t n_pq = 2 * (size_t)A.nbA, n_r = 2 * (2 * (size_t)A.nbB + 8 * B), n_c = 2 * 7 * (size_t)T.K;
+    const size_t nw = n_pq + n_r + n_c;
+    const unsigned long long* had = L.team_words.p;
+    unsigned long long* w = L.team_words.ensure(nw, s);
+    if (w != had || L.team_tag > 0xffffffffull - (unsigned long long)A.maxit - 2) {
+        IDP_LAUNCH(k_zero_words, grid_for((long)L.team_words.cap, 256), 256, 0, s, (long)L.team_words.cap, w);
+        L.team_tag = 0;
+    }
+    T.w_pq = w;
+    T.w_r = w + n_pq;
+    T.w_rc = T.w_r + n_r;
+    T.w_cp = T.w_rc + 12 * (size_t)T.K;
+    T.tag0 = (unsigned)L.team_tag;
+    L.team_tag += (unsigned long long)A.maxit + 2;
+    T.ctl = team;
+    T.done = team + 3;
+    T.nstart = handover ? nrun : 0;
+    T.spin_limit = 1L << 23;
+    T.aptr = L.coarse.aptr.p;
+    T.avert = L.coarse.avert.p;
+    T.Ps = L.coarse.Ps.p;
+    T.Ainv = L.coarse.Ainv.p;
+    static const void* const fns[] = {(const void*)k_pcg_team<false, false>, (const void*)k_pcg_team<false, true>,
+                                      (const void*)k_pcg_team<true, false>, (const void*)k_pcg_team<true, true>};
+    const void* fn = fns[(one ? 2 : 0) + (coarse ? 1 : 0)];
+    PcgArgs a = A;
+    void* args[] = {&a, &T};
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    L.team_tok = L.prof ? L.prof->pair(e0, e1) : -1;
+    if (e0) IDP_HIP(hipEventRecord(e0, s));
+    // workgroups that wait for each other have to be resident together
+    if (one) IDP_HIP(hipLaunchKernel(fn, dim3(tab.size()), dim3(TEAM_THREADS), args, 0, s));
+    else IDP_HIP(hipLaunchCooperativeKernel(fn, dim3(tab.size()), dim3(TEAM_THREADS), args, 0, s));
+    if (e1) IDP_HIP(hipEventRecord(e1, s));
+    return true;
 }
 
 // Preconditioned CG per instance on the assembled system (E + C); b, x: 3V.
@@ -1357,7 +2192,10 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     const double nnzb = (double)m.nnzb_e + (double)L.ncb;
     int* err = L.err.ensure(2 * (size_t)B + 2, s);
     int* flag = err + B;
-    IDP_LAUNCH(k_pcg_start, grid_for(B, 64), 64, 0, s, B, solve, flag, err);
+    // team kernel: control words and per-instance hand-over counts
+    const int nteam = 3 + B;
+    int* team = L.team.ensure(nteam, s);
+    IDP_LAUNCH(k_pcg_start, grid_for(std::max(B, nteam), 256), 256, 0, s, B, solve, flag, err, nteam, team);
     const bool haveC = L.ncb > 0;
     Profiler* P = L.prof;
     const int tok = P ? P->begin(IDP_K_PCG) : -1;
@@ -1507,9 +2345,19 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     // their state for the next call.  One solve alone is never handed over.
     int nstart = 0;
     for (int i = 0; i < B; ++i) nstart += run[i];
+    std::vector<int> hdone(B, 0);
+    const bool teamed = nA > 0 && !A.red && shape.g == 8 && pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
+    if (teamed) {
+        std::vector<int> ht(3 + B);
+        IDP_HIP(hipMemcpyAsync(hf.data(), err, 2 * B * sizeof(int), hipMemcpyDeviceToHost, s));
+        IDP_HIP(hipMemcpyAsync(ht.data(), team, ht.size() * sizeof(int), hipMemcpyDeviceToHost, s));
+        IDP_HIP(hipStreamSynchronize(s));
+        if (ht[0]) throw HipError(IDP_E_HIP, "PCG: a workgroup's wait for its team ran out");
+        for (int i = 0; i < B; ++i) hdone[i] = ht[3 + i];
+    }
     int it_half = -1, it_end = INT_MAX;
     int it = 0, chunk = 8;
-    for (; nA > 0 && it < it_end;) {
+    for (; !teamed && nA > 0 && it < it_end;) {
         for (int j = 0; j < chunk && it <= maxit && it < it_end; ++j, ++it) {
             // kernel times (events recorded by the dispatch itself) on one
             // iteration in 8
@@ -1556,10 +2404,11 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         iters[i] = 0;
         relres[i] = 0;
         if (f == 0) {
-            if (it < it_end) throw HipError(IDP_E_HIP, "PCG did not stop");
+            const int did = teamed ? hdone[i] : it;
+            if (teamed ? did == 0 : it < it_end) throw HipError(IDP_E_HIP, "PCG did not stop");
             iters[i] = PCG_HANDED_OVER;  // continues in the next call
-            L.h_it0[i] += it;
-            maxdone = std::max(maxdone, it);
+            L.h_it0[i] += did;
+            maxdone = std::max(maxdone, did);
             continue;
         }
         if (f == 3) continue;
@@ -1575,6 +2424,14 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         }
     }
     if (P) {
+        if (teamed) {  // the whole solve as one launch: the bytes of all its iterations
+            double w = 0.0;
+            for (int i = 0; i < B; ++i) {
+                const int k = hf[B + i] == 0 ? hdone[i] : hf[B + i] == 3 ? 0 : (int)hs[3 * i + 2] - L.h_it0[i];
+                w += (spmv_bytes + upd_bytes) * k * (double)(I.vbeg[i + 1] - I.vbeg[i]) / std::max(nV, 1);
+            }
+            P->end_pair(IDP_K_PCG_SPMV, L.team_tok, w);
+        }
         // launches at or after the last stopping iteration did no work
         P->discard_from(IDP_K_PCG_SPMV, maxdone);
         P->discard_from(IDP_K_PCG_UPDATE, maxdone);

@@ -14,10 +14,10 @@ struct CoarseWork {
     bool ready = false;     // a level exists (built for this mesh and Dirichlet set)
     int age = 0, nV = 0;
     const unsigned char* mask = nullptr;  // the Dirichlet mask it was built with
-    int K = 0, ncd = 0, nsb = 0;
+    int K = 0, ncd = 0, nsb = 0, nfree = 0;
     DBuf<int> agg, aptr, avert;
     DBuf<double> P, Ainv, rc, part;
-    DBuf<double> Ps;  // P in aggregate order (18 doubles per slot of avert)
+    DBuf<double> Ps;  // P in aggregate order: 18 planes over the slots of avert
     DBuf<unsigned long long> key0, key1;
     DBuf<unsigned> val0, val1, head, hs, seg;
     DBuf<unsigned char> tmp;
@@ -53,6 +53,11 @@ struct LinWork {
     // PCG
     DBuf<double> pinv, r, z, p, p1, q, part0, part1, part2, part3, part_bx, scal, scal2, red;
     DBuf<int> err;
+    DBuf<int> team, team_it0;  // words of the one-kernel solve, iterations of earlier calls
+    DBuf<int4> team_tab;
+    DBuf<unsigned long long> team_words;
+    unsigned long long team_tag = 0;  // last tag used in them
+    int team_tok = -1;                // profiler token of the last one-kernel solve
     // cluster preconditioner
     DBuf<int> cl_best, cl_root, cl_size, cl_root2, cl_cnt, cl_mem, cl_cm4;
     DBuf<unsigned long long> cl_pack;

@@ -112,7 +112,8 @@ enum {
     IDP_K_CCD = 5,          /* ACCD kernel over candidate pairs (pair count) */
     IDP_K_ENERGY = 6,       /* tet + inertia + barrier energy kernels */
     IDP_K_GRADIENT = 7,     /* tet + barrier gradient and vertex gather */
-    IDP_K_PCG_SPMV = 8,     /* PCG SpMV kernel, sampled on one iteration in 8 (bytes) */
+    IDP_K_PCG_SPMV = 8,     /* PCG SpMV kernel, sampled on one iteration in 8, or the whole solve where it
+                               runs as one kernel (bytes) */
     IDP_K_PCG_UPDATE = 9,   /* PCG vector-update kernel, sampled likewise (bytes) */
     IDP_K_FRICTION = 10,    /* friction Hessian kernel (bytes) */
     IDP_K_FRICTION_BASIS = 11, /* friction basis update: flags, scan, records (bytes) */

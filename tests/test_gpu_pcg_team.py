@@ -1,0 +1,81 @@
+"""The PCG solve as one kernel on MI355X: its sums are formed in the order of
+the two-kernel loop, so a Newton direction is the same bit for bit whichever
+runs it.  A batch of more rows than one launch holds takes the two-kernel
+loop."""
+import numpy as np
+import pytest
+
+from idp_amd import driver, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def _scene(nx, ny, nz, seed=5):
+    X, tets = scenes.kuhn_block(nx, ny, nz, 0.05)
+    rng = np.random.default_rng(seed)
+    X = X + rng.normal(0.0, 0.001, X.shape)
+    side = 0.05 * min(nx, ny, nz)
+    return scenes.Scene(f"bar{nx}x{ny}x{nz}", X, tets, scenes.sinusoid_target(X, side, 4, (0.2, 0.4), (0.5, 1.0), rng))
+
+
+# rows of the first instance: 8 (less than a wavefront's), 64 and 66 (one
+# 64-row block, one and two rows more), 126 and 130 (one workgroup and the
+# next), 195 (odd number of 64-row blocks, two workgroups)
+@pytest.mark.parametrize("cells", [(1, 1, 1), (3, 3, 3), (10, 2, 1), (6, 5, 2), (12, 4, 1), (12, 4, 2)])
+def test_one_kernel_equals_two_kernels(cells):
+    sc = _scene(*cells)
+    big = _scene(31, 31, 31, seed=6)  # 32,768 rows: the batch no longer fits one launch
+    a, b = driver.BatchAnimFix([sc]), driver.BatchAnimFix([sc, big])
+    try:
+        say(f"[pcg team] {sc.X.shape[0]} rows alone, then beside {big.X.shape[0]}")
+        a.advance_one_time_step(max_newton=2)
+        b.advance_one_time_step(max_newton=2)
+        Xa, va = a.state(0)
+        Xb, vb = b.state(0)
+        assert np.array_equal(Xa, Xb) and np.array_equal(va, vb)
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("cells,verts", [((20, 4, 4), 48), ((33, 9, 7), 144), ((64, 16, 16), 144), ((40, 40, 1), 64)])
+def test_one_kernel_with_coarse_level(cells, verts):
+    """The direction agrees with the one without a coarse level to the solves'
+    residual, and a second solve of the same system gives the same bits."""
+    sc = _scene(*cells)
+    d = driver.TetAnimFix(sc)
+    try:
+        def direction(cv):
+            return d.ctx.newton_direction(sc.X, sc.target, sc.h, d.dHat2, d.kappa[0], pcg_rtol=1e-10, coarse_verts=cv)
+
+        g0, s0, r0, i0 = direction(-1)
+        g1, s1, r1, i1 = direction(verts)
+        g2, s2, r2, i2 = direction(verts)
+        say(f"[pcg team] {sc.X.shape[0]} rows: {i0} iterations without the coarse level, {i1} with it")
+        assert r0 <= 1e-10 and r1 <= 1e-10
+        assert np.array_equal(g0, g1) and np.array_equal(s1, s2) and i1 == i2
+        # |error| <= cond |residual|: 1e-8 holds for systems of condition below 100
+        assert np.linalg.norm(s1 - s0) <= 1e-8 * np.linalg.norm(s0)
+    finally:
+        d.close()
+
+
+def test_batch_of_many_small_meshes_in_one_kernel():
+    """Instances of one workgroup each and of several, together and alone."""
+    mix = [scenes.cube_sinusoid(n, seed=n) for n in (2, 4, 5, 3, 6, 8, 4, 2)]
+    b = driver.BatchAnimFix(mix)
+    its, _ = b.advance_one_time_step(max_newton=4)
+    for i, sc in enumerate(mix):
+        say(f"[pcg team] instance {i} alone ({sc.X.shape[0]} rows)")
+        a = driver.BatchAnimFix([sc])
+        ia, _ = a.advance_one_time_step(max_newton=4)
+        assert ia[0] == its[i]
+        Xa, va = a.state(0)
+        Xm, vm = b.state(i)
+        assert np.array_equal(Xa, Xm) and np.array_equal(va, vm)
+        a.close()
+    b.close()
