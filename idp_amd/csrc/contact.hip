@@ -124,22 +124,49 @@ __global__ void __launch_bounds__(256) k_edge_len_parts(const int* __restrict__ 
 // sum of |p| over an instance's boundary nodes, x, y, z of each node in node
 // order, one add after another: the order of the reference's loop
 // (SPATIAL_HASH.h:466-474), so the span cap rounds as it does there.  One
-// thread per instance; the loads run ahead of the dependent adds.
-__global__ void k_psize_seq(int B, const int* __restrict__ nbeg, const int* __restrict__ bn,
-                            const double* __restrict__ p, double* __restrict__ out,
-                            const unsigned char* __restrict__ active)
+// workgroup per instance: wavefront 0 adds one tile of values from LDS while
+// the others load the next, so the serial chain is the adds alone (35,330
+// nodes with the loads in the chain: 2,631 us).
+constexpr int PSIZE_TILE = 768;  // nodes of a tile (2 x 18 KB of LDS)
+__global__ void __launch_bounds__(256) k_psize_seq(int B, const int* __restrict__ nbeg, const int* __restrict__ bn,
+                                                   const double* __restrict__ p, double* __restrict__ out,
+                                                   const unsigned char* __restrict__ active)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double buf[2][3 * PSIZE_TILE];
+    const int i = blockIdx.x;
     if (i >= B || (active && !active[i])) return;
+    const int b = nbeg[i], n = nbeg[i + 1] - b;
+    auto load = [&](int t, int first, int step) {
+        const int m = min(PSIZE_TILE, n - t * PSIZE_TILE);
+        for (int k = first; k < m; k += step) {
+            const int v = bn[b + t * PSIZE_TILE + k];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) buf[t & 1][3 * k + d] = fabs(p[3 * v + d]);
+        }
+    };
+    const int nt = (n + PSIZE_TILE - 1) / PSIZE_TILE;
+    if (nt) load(0, threadIdx.x, 256);
+    __syncthreads();
     double ps = 0.0;
-#pragma unroll 8
-    for (int k = nbeg[i]; k < nbeg[i + 1]; ++k) {
-        const int v = bn[k];
-        ps += fabs(p[3 * v]);
-        ps += fabs(p[3 * v + 1]);
-        ps += fabs(p[3 * v + 2]);
+    for (int t = 0; t < nt; ++t) {
+        if (threadIdx.x >= 64) {
+            if (t + 1 < nt) load(t + 1, threadIdx.x - 64, 192);
+        } else {
+            const int m = 3 * min(PSIZE_TILE, n - t * PSIZE_TILE);
+            const double* q = buf[t & 1];
+            int k = 0;
+            for (; k + 16 <= m; k += 16) {
+                double v[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) v[u] = q[k + u];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) ps += v[u];
+            }
+            for (; k < m; ++k) ps += q[k];
+        }
+        __syncthreads();
     }
-    out[i] = ps;
+    if (threadIdx.x == 0) out[i] = ps;
 }
 
 // min / max of positions (and of x + alpha_i p when p is given) over the
@@ -437,9 +464,20 @@ __device__ inline unsigned long long ee_pass_key(const CSOut& O, int inst, int e
            ((unsigned long long)(eI - O.ebeg[inst]) * ne + (unsigned long long)(eJ - O.ebeg[inst]));
 }
 
+// one slot for each lane of the wavefront that calls this together: a single
+// atomic on the counter, whose address all lanes share
+__device__ inline unsigned append_slot(unsigned* ctr)
+{
+    const unsigned long long m = __ballot(1);
+    const int lane = threadIdx.x & 63, leader = __ffsll((long long)m) - 1;
+    unsigned base = 0;
+    if (lane == leader) base = atomicAdd(ctr, (unsigned)__popcll(m));
+    return __shfl(base, leader) + (unsigned)__popcll(m & ((1ull << lane) - 1));
+}
+
 __device__ inline void out_pass(const CSOut& O, unsigned long long key, int a, int b, int c, int d)
 {
-    const unsigned i = atomicAdd(O.cnt, 1u);
+    const unsigned i = append_slot(O.cnt);
     if (i < O.cap_p) {
         O.pkey[i] = key;
         O.pval[i] = make_int4(a, b, c, d);
@@ -450,7 +488,7 @@ __device__ inline void out_pass(const CSOut& O, unsigned long long key, int a, i
 // in std::map order, over instance-local vertex ids
 __device__ inline void out_dup(const CSOut& O, int inst, int a, int b, int c)
 {
-    const unsigned i = atomicAdd(O.cnt + 1, 1u);
+    const unsigned i = append_slot(O.cnt + 1);
     if (i < O.cap_d) {
         const long long vb = O.vbeg[inst];
         const unsigned long long V = (unsigned long long)(O.vbeg[inst + 1] - vb);
@@ -986,13 +1024,25 @@ __global__ void __launch_bounds__(256) k_accd(const unsigned* __restrict__ cnt, 
     bool active = false, finished = false;
     int steps = 0, slice = 0;
     double amin_pf = 0.0;  // running minimum of this lane's instance, loaded ahead of use
+    // a lane's first pair is its own index; the queue counter starts after all
+    // lanes' first pairs, so a launch of few pairs costs no atomics (one per
+    // wavefront of the grid on one address took 100 us)
+    bool first = true;
+    const unsigned lanes = gridDim.x * blockDim.x;
     for (;;) {
         const unsigned long long idle = __ballot(!active && !finished);
         if (idle) {
             const int leader = __ffsll((long long)idle) - 1;
             unsigned base = 0;
-            if (lane == leader) base = atomicAdd(next, (unsigned)__popcll(idle));
-            base = __shfl(base, leader);
+            if (first) {  // the whole wavefront is idle
+                base = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u;
+                first = false;
+            } else if (n <= lanes) {
+                base = n;  // every pair was some lane's first
+            } else {
+                if (lane == leader) base = lanes + atomicAdd(next, (unsigned)__popcll(idle));
+                base = __shfl(base, leader);
+            }
             if (!active && !finished) {
                 const unsigned j = base + (unsigned)__popcll(idle & ((1ull << lane) - 1));
                 slice = 0;
@@ -1476,7 +1526,7 @@ void contact_ccd_batch(ContactWork& w, hipStream_t s, const MeshDev& m, const do
     double* ep = w.dparts.ensure(I.echunk.nblk + B + 2, s);
     double* pp = ep + I.echunk.nblk + 1;
     IDP_LAUNCH(k_edge_len_parts, I.echunk.nblk, 256, 0, s, I.echunk.lo.p, I.echunk.hi.p, (const int2*)m.be.p, X, ep);
-    IDP_LAUNCH(k_psize_seq, grid_for(B, 64), 64, 0, s, B, I.d_nbeg.p, m.bn.p, P, pp, active);
+    IDP_LAUNCH(k_psize_seq, B, 256, 0, s, B, I.d_nbeg.p, m.bn.p, P, pp, active);
     double* ain = (double*)w.scal2.ensure(2 * (size_t)B + 4, s);
     IDP_HIP(hipMemcpyAsync(ain, alpha_io, B * sizeof(double), hipMemcpyHostToDevice, s));
     double* dalpha = w.ialpha.ensure(B, s);
