@@ -282,13 +282,20 @@ struct ClElastic {
     long ld;
 };
 
+// The rows of the two matching passes are read by groups of CL_LANES lanes,
+// neighbouring lanes taking neighbouring blocks, so that a plane's loads
+// share lines (one lane per row: 94 us a pass on the 64x16x16 bar, 800 us on
+// 386,561 rows).
+constexpr int CL_LANES = 8;
+
 // strongest contact neighbour of every vertex (ties: smaller id); -1 if none
 __global__ void k_cl_best(int nV, const int* __restrict__ crp, const int* __restrict__ ccol,
                           const double* __restrict__ cval, long cld, ClElastic el, ClMask cm,
                           int* __restrict__ best)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nV || cm.skip(v)) return;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = (int)(t / CL_LANES), lane = (int)(t % CL_LANES);
+    if (v >= nV || cm.skip(v)) return;  // uniform over the group
     int b = -1;
     double bw = 0.0;
     auto consider = [&](int u, double w) {
@@ -298,10 +305,20 @@ __global__ void k_cl_best(int nV, const int* __restrict__ crp, const int* __rest
         }
     };
     if (crp)
-        for (int k = crp[v]; k < crp[v + 1]; ++k) consider(ccol[k], cblock_norm2(cval, cld, k));
+        for (int k = crp[v] + lane; k < crp[v + 1]; k += CL_LANES) consider(ccol[k], cblock_norm2(cval, cld, k));
     if (el.rp)
-        for (int k = el.rp[v]; k < el.rp[v + 1]; ++k) consider(el.col[k], cblock_norm2(el.val, el.ld, k));
-    best[v] = b;
+        for (int k = el.rp[v] + lane; k < el.rp[v + 1]; k += CL_LANES)
+            consider(el.col[k], cblock_norm2(el.val, el.ld, k));
+#pragma unroll
+    for (int o = CL_LANES / 2; o > 0; o >>= 1) {
+        const int u = __shfl_xor(b, o, CL_LANES);
+        const double w = __shfl_xor(bw, o, CL_LANES);
+        if (u >= 0 && (w > bw || (w == bw && (b < 0 || u < b)))) {
+            bw = w;
+            b = u;
+        }
+    }
+    if (lane == 0) best[v] = b;
 }
 
 __global__ void k_cl_pair(int nV, const int* __restrict__ best, ClMask cm, int* __restrict__ root,
@@ -324,8 +341,9 @@ __global__ void k_cl_best2(int nV, const int* __restrict__ crp, const int* __res
                            const int* __restrict__ size, ClElastic el, ClMask cm,
                            unsigned long long* __restrict__ pack)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nV || (!crp && !el.rp) || cm.skip(v)) return;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = (int)(t / CL_LANES), lane = (int)(t % CL_LANES);
+    if (v >= nV || (!crp && !el.rp) || cm.skip(v)) return;  // uniform over the group
     const int r = root[v];
     unsigned long long bestp = 0;
     auto consider = [&](int u, double w) {
@@ -337,10 +355,16 @@ __global__ void k_cl_best2(int nV, const int* __restrict__ crp, const int* __res
         if (p > bestp) bestp = p;
     };
     if (crp)
-        for (int k = crp[v]; k < crp[v + 1]; ++k) consider(ccol[k], cblock_norm2(cval, cld, k));
+        for (int k = crp[v] + lane; k < crp[v + 1]; k += CL_LANES) consider(ccol[k], cblock_norm2(cval, cld, k));
     if (el.rp)
-        for (int k = el.rp[v]; k < el.rp[v + 1]; ++k) consider(el.col[k], cblock_norm2(el.val, el.ld, k));
-    if (bestp) atomicMax(pack + r, bestp);
+        for (int k = el.rp[v] + lane; k < el.rp[v + 1]; k += CL_LANES)
+            consider(el.col[k], cblock_norm2(el.val, el.ld, k));
+#pragma unroll
+    for (int o = CL_LANES / 2; o > 0; o >>= 1) {
+        const unsigned long long p = __shfl_xor(bestp, o, CL_LANES);
+        bestp = p > bestp ? p : bestp;
+    }
+    if (lane == 0 && bestp) atomicMax(pack + r, bestp);
 }
 
 __global__ void k_cl_merge(int nV, int* __restrict__ root, const unsigned long long* __restrict__ pack,
@@ -388,32 +412,54 @@ __global__ void k_cl_sort(int nV, const int* __restrict__ root, const int* __res
     }
 }
 
-// locate block (a, b) in a BSR row; returns -1 when absent
+// locate block (a, b) in a BSR row; returns -1 when absent (8 columns are
+// read together)
 __device__ inline int bsr_find(const int* __restrict__ rp, const int* __restrict__ col, int a, int b)
 {
-    for (int k = rp[a]; k < rp[a + 1]; ++k)
-        if (col[k] == b) return k;
-    return -1;
+    const int e = rp[a + 1];
+    int f = -1;
+    for (int k = rp[a]; k < e && f < 0; k += 8) {
+        int c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = col[min(k + u, e - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (k + u < e && c[u] == b) f = k + u;
+    }
+    return f;
 }
 
-// one thread per cluster root: gather the (3k)^2 block of E + C, Cholesky,
-// inverse, and scatter the member rows to Z.  Singletons keep the 3x3 inverse
-// of the block-Jacobi preconditioner (same arithmetic).
-__global__ void k_cl_build(int nV, const int* __restrict__ root, const int* __restrict__ cnt,
-                           const int* __restrict__ mem, const int* __restrict__ ediag,
-                           const int* __restrict__ erp, const int* __restrict__ ecol, const double* __restrict__ evals,
-                           long eld, const int* __restrict__ cdiag, const int* __restrict__ crp,
-                           const int* __restrict__ ccol, const double* __restrict__ cvals, long cld,
-                           const int* __restrict__ vinst, ClMask cmask, double* __restrict__ Z,
-                           int4* __restrict__ cm4, double* __restrict__ work, int* __restrict__ err)
+// Gathers a cluster's (3k)^2 block of E + C, factors it (Cholesky), inverts
+// it and scatters the member rows to Z, by 16 lanes per vertex (the group of
+// the cluster's root works): lane 4a + b gathers the 3x3 block of members a
+// and b, lane i holds row i of the factorization, lane c forms column c of the
+// inverse.  The factor is padded to order 12 with the identity, so every loop
+// is unrolled and the rows stay in registers; each entry is formed by the same
+// operations in the same order as a sequential Cholesky.  One thread per
+// cluster with its matrices in memory took 157 us on 81 rows and 370 us on
+// 18,785 (a chain of dependent loads).  Singletons keep the 3x3 inverse of the
+// block-Jacobi preconditioner (same arithmetic).
+constexpr int CL_N = 3 * CL_MAX;
+__global__ void __launch_bounds__(256) k_cl_build(
+    int nV, const int* __restrict__ root, const int* __restrict__ cnt, const int* __restrict__ mem,
+    const int* __restrict__ ediag, const int* __restrict__ erp, const int* __restrict__ ecol,
+    const double* __restrict__ evals, long eld, const int* __restrict__ cdiag, const int* __restrict__ crp,
+    const int* __restrict__ ccol, const double* __restrict__ cvals, long cld, const int* __restrict__ vinst, ClMask cmask,
+    double* __restrict__ Z, int4* __restrict__ cm4, int* __restrict__ err)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nV || cmask.skip(r) || root[r] != r) return;
-    const int k = min(cnt[r], CL_MAX);
-    const int* m = mem + CL_MAX * r;
-    const int4 list = make_int4(m[0], k > 1 ? m[1] : -1, k > 2 ? m[2] : -1, k > 3 ? m[3] : -1);
-    for (int a = 0; a < k; ++a) cm4[m[a]] = list;
-    if (k == 1) {
+    __shared__ double sh[16][CL_N][CL_N + 1];
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = (int)(t >> 4), g = (int)(t & 15);
+    double(*M)[CL_N + 1] = sh[threadIdx.x >> 4];
+    // uniform over the group of 16 lanes
+    const bool work = r < nV && !cmask.skip(r) && root[r] == r;
+    const int k = work ? min(cnt[r], CL_MAX) : 0;
+    const int* m = mem + CL_MAX * (size_t)min(r, nV - 1);
+    int mm[CL_MAX];
+#pragma unroll
+    for (int a = 0; a < CL_MAX; ++a) mm[a] = a < k ? m[a] : -1;
+    if (work && g < k) cm4[m[g]] = make_int4(mm[0], mm[1], mm[2], mm[3]);
+    if (k == 1 && g == 0) {
         double a[9];
         const long ed = ediag[r];
 #pragma unroll
@@ -441,74 +487,88 @@ __global__ void k_cl_build(int nV, const int* __restrict__ root, const int* __re
         o[2] = (a[1] * a[5] - a[2] * a[4]) * id;
         o[5] = (a[2] * a[3] - a[0] * a[5]) * id;
         o[8] = (a[0] * a[4] - a[1] * a[3]) * id;
-        return;
     }
-    const int n = 3 * k;
-    double* A = work + (size_t)2 * 144 * r;  // n x n, row-major
-    double* Ainv = A + 144;
-    for (int a = 0; a < k; ++a)
-        for (int b = 0; b < k; ++b) {
-            double blk[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const bool big = k > 1;
+    // ---- gather
+    {
+        const int a = g >> 2, b = g & 3;
+        double blk[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) blk[i] = (a == b && i % 4 == 0 && a >= k) ? 1.0 : 0.0;
+        if (big && a < k && b < k) {
             const int ke = bsr_find(erp, ecol, m[a], m[b]);
             if (ke >= 0)
+#pragma unroll
                 for (int i = 0; i < 9; ++i) blk[i] += evals[i * eld + ke];
             if (crp) {
                 const int kc = bsr_find(crp, ccol, m[a], m[b]);
                 if (kc >= 0)
+#pragma unroll
                     for (int i = 0; i < 9; ++i) blk[i] += cvals[i * cld + kc];
             }
-            for (int i = 0; i < 3; ++i)
-                for (int j = 0; j < 3; ++j) A[(3 * a + i) * n + 3 * b + j] = blk[3 * i + j];
         }
-    // symmetrise (the assembled blocks are symmetric up to rounding) and factor A = L L^T in place
-    for (int i = 0; i < n; ++i)
-        for (int j = 0; j < i; ++j) {
-            const double sym = 0.5 * (A[i * n + j] + A[j * n + i]);
-            A[i * n + j] = sym;
-            A[j * n + i] = sym;
-        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) M[3 * a + i][3 * b + j] = blk[3 * i + j];
+    }
+    __syncthreads();
+    // ---- row i of the lower triangle, symmetrised (the assembled blocks are
+    // symmetric up to rounding), factored column by column
+    const int row = min(g, CL_N - 1);
+    double L[CL_N];
+#pragma unroll
+    for (int j = 0; j < CL_N; ++j) L[j] = j == row ? M[row][j] : 0.5 * (M[row][j] + M[j][row]);
     bool ok = true;
-    for (int j = 0; j < n && ok; ++j) {
-        double d = A[j * n + j];
-        for (int q = 0; q < j; ++q) d -= A[j * n + q] * A[j * n + q];
-        if (!(d > 0)) {
-            ok = false;
-            break;
-        }
-        const double ljj = sqrt(d);
-        A[j * n + j] = ljj;
-        for (int i = j + 1; i < n; ++i) {
-            double t = A[i * n + j];
-            for (int q = 0; q < j; ++q) t -= A[i * n + q] * A[j * n + q];
-            A[i * n + j] = t / ljj;
-        }
+#pragma unroll
+    for (int q = 0; q < CL_N; ++q) {
+        const double d = __shfl(L[q], q, 16);
+        ok = ok && d > 0;
+        const double lqq = sqrt(d);
+        L[q] = row == q ? lqq : L[q] / lqq;
+#pragma unroll
+        for (int j = q + 1; j < CL_N; ++j) L[j] -= L[q] * __shfl(L[q], j, 16);
+    }
+    __syncthreads();  // every lane has read M
+    if (g < CL_N)
+#pragma unroll
+        for (int j = 0; j < CL_N; ++j)
+            if (j <= g) M[g][j] = L[j];
+    __syncthreads();
+    if (!big) return;
+    // ---- column c of the inverse: L y = e_c, L^T x = y
+    const int c = row;
+    double y[CL_N];
+#pragma unroll
+    for (int i = 0; i < CL_N; ++i) {
+        double s = i == c ? 1.0 : 0.0;
+#pragma unroll
+        for (int q = 0; q < i; ++q) s -= M[i][q] * y[q];
+        y[i] = s / M[i][i];
+    }
+#pragma unroll
+    for (int i = CL_N - 1; i >= 0; --i) {
+        double s = y[i];
+#pragma unroll
+        for (int q = i + 1; q < CL_N; ++q) s -= M[q][i] * y[q];
+        y[i] = s / M[i][i];
     }
     if (!ok) {
-        atomicOr(err + vinst[r], 1);
-        for (int i = 0; i < n * n; ++i) Ainv[i] = (i % (n + 1)) == 0 ? 1.0 : 0.0;
-    } else {
-        // inverse column by column: solve L y = e_c, L^T x = y
-        for (int c = 0; c < n; ++c) {
-            double y[12];
-            for (int i = 0; i < n; ++i) {
-                double t = (i == c) ? 1.0 : 0.0;
-                for (int q = 0; q < i; ++q) t -= A[i * n + q] * y[q];
-                y[i] = t / A[i * n + i];
-            }
-            for (int i = n - 1; i >= 0; --i) {
-                double t = y[i];
-                for (int q = i + 1; q < n; ++q) t -= A[q * n + i] * Ainv[q * n + c];
-                Ainv[i * n + c] = t / A[i * n + i];
-            }
-        }
+        if (g == 0) atomicOr(err + vinst[r], 1);
+#pragma unroll
+        for (int i = 0; i < CL_N; ++i) y[i] = i == c ? 1.0 : 0.0;
     }
-    // member a's rows, as k 3x3 blocks: block (a, b) in plane b at row m[a]
-    for (int a = 0; a < k; ++a)
-        for (int b = 0; b < k; ++b) {
-            double* o = Z + 9 * ((size_t)b * nV + m[a]);
-            for (int i = 0; i < 3; ++i)
-                for (int j = 0; j < 3; ++j) o[3 * i + j] = Ainv[(3 * a + i) * n + 3 * b + j];
-        }
+    // ---- member a's rows, as k 3x3 blocks: block (a, b) in plane b at row m[a]
+    if (g < 3 * k) {
+        const int b = g / 3, j = g % 3;
+#pragma unroll
+        for (int a = 0; a < CL_MAX; ++a)
+            if (a < k) {
+                double* o = Z + 9 * ((size_t)b * nV + mm[a]);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) o[3 * i + j] = y[3 * a + i];
+            }
+    }
 }
 
 // z_v = Z_v r_members (members' r given by rfun).  Z holds CL_MAX planes of
@@ -2217,18 +2277,18 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     const ClElastic elm{L.precond == 0 ? m.e_rowptr.p : nullptr, m.e_col.p, L.evals.p, m.nnzb_e};
     // only the instances that solve (new or continued) build their clusters
     const ClMask cmk{I.vinst.p, solve};
-    IDP_LAUNCH(k_cl_best, vg, 256, 0, s, nV, crp_match, L.ccol.p, L.cvals.p, L.ncb, elm, cmk, best);
+    const int vgl = grid_for((long)CL_LANES * nV, 256);
+    IDP_LAUNCH(k_cl_best, vgl, 256, 0, s, nV, crp_match, L.ccol.p, L.cvals.p, L.ncb, elm, cmk, best);
     IDP_LAUNCH(k_cl_pair, vg, 256, 0, s, nV, best, cmk, root, size);
     IDP_HIP(hipMemsetAsync(pack, 0, nV * sizeof(unsigned long long), s));
-    IDP_LAUNCH(k_cl_best2, vg, 256, 0, s, nV, crp_match, L.ccol.p, L.cvals.p, L.ncb, root, size, elm, cmk, pack);
+    IDP_LAUNCH(k_cl_best2, vgl, 256, 0, s, nV, crp_match, L.ccol.p, L.cvals.p, L.ncb, root, size, elm, cmk, pack);
     IDP_LAUNCH(k_cl_merge, vg, 256, 0, s, nV, root, pack, size, cmk, root2);
     IDP_HIP(hipMemsetAsync(cnt, 0, nV * sizeof(int), s));
     IDP_LAUNCH(k_cl_members, vg, 256, 0, s, nV, root2, cmk, cnt, mem);
     IDP_LAUNCH(k_cl_sort, vg, 256, 0, s, nV, root2, cnt, cmk, mem);
-    double* work = L.cl_work.ensure(2 * 144 * (size_t)nV, s);
-    IDP_LAUNCH(k_cl_build, vg, 256, 0, s, nV, root2, cnt, mem, m.e_diag.p, m.e_rowptr.p, m.e_col.p, L.evals.p,
+    IDP_LAUNCH(k_cl_build, grid_for(16L * nV, 256), 256, 0, s, nV, root2, cnt, mem, m.e_diag.p, m.e_rowptr.p, m.e_col.p, L.evals.p,
                m.nnzb_e, haveC ? L.cdiag.p : (const int*)nullptr, crp, L.ccol.p, L.cvals.p, L.ncb, I.vinst.p, cmk, Z,
-               cm4, work, err);
+               cm4, err);
     // coarse level: one instance with the positions of its system given
     const bool coarse = B == 1 && L.xpos && L.coarse.verts_per_agg > 0 && sv[0] == 1 && coarse_setup(L, s, m, L.xpos);
     PcgArgs A;

@@ -61,7 +61,6 @@ struct LinWork {
     // cluster preconditioner
     DBuf<int> cl_best, cl_root, cl_size, cl_root2, cl_cnt, cl_mem, cl_cm4;
     DBuf<unsigned long long> cl_pack;
-    DBuf<double> cl_work;
     Profiler* prof = nullptr;
     CoarseWork coarse;
     const double* xpos = nullptr;  // positions of the system being solved (coarse aggregation); null: none
