@@ -1248,7 +1248,7 @@ struct TeamArgs {
     int nstart;       // hand-over: solves at launch (0: never)
     long spin_limit;  // polls of one wait at most
     // coarse level (one instance; K = 0: none)
-    int K, ncd, nfree;
+    int K, ncd, lda, nfree;
     const int *aptr, *avert;
     const double *Ps, *Ainv;
 };
@@ -1882,12 +1882,12 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
                 const int a = a0 + q4 * size;
                 double e[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
                 if (a < T.K) {
-                    const double* Ar = T.Ainv + (size_t)(6 * a) * T.ncd;
+                    const double* Ar = T.Ainv + (size_t)(6 * a) * T.lda;
 #pragma unroll 4
                     for (int j = t4; j < T.ncd; j += 256) {
                         const double rj = val[j];
 #pragma unroll
-                        for (int m = 0; m < 6; ++m) e[m] += Ar[(size_t)m * T.ncd + j] * rj;
+                        for (int m = 0; m < 6; ++m) e[m] += Ar[(size_t)m * T.lda + j] * rj;
                     }
                 }
 #pragma unroll
@@ -2190,6 +2190,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     T.K = coarse ? L.coarse.K : 0;
     T.ncd = L.coarse.ncd;
     T.nfree = L.coarse.nfree;
+    T.lda = L.coarse.lda;
     if (T.K && (T.ncd > TEAM_VALUES || T.K > TEAM_TASKS)) return false;
     // published words; tags only grow, so words of earlier launches never match (cleared when they would wrap)
     const size_t n_pq = 2 * (size_t)A.nbA, n_r = 2 * (2 * (size_t)A.nbB + 8 * B), n_c = 2 * 7 * (size_t)T.K;

@@ -14,20 +14,15 @@ struct CoarseWork {
     bool ready = false;     // a level exists (built for this mesh and Dirichlet set)
     int age = 0, nV = 0;
     const unsigned char* mask = nullptr;  // the Dirichlet mask it was built with
-    int K = 0, ncd = 0, nsb = 0, nfree = 0;
+    int K = 0, ncd = 0, lda = 0, nsb = 0, nfree = 0;  // lda: leading dimension of A_c^-1
     DBuf<int> agg, aptr, avert;
-    DBuf<double> P, Ainv, rc, part;
+    DBuf<double> P, Ainv, Awork, diag, box, rc, part;
+    DBuf<unsigned> ckey0, ckey1, cval0, cval1, ccnt;  // voxels of the vertices
     DBuf<double> Ps;  // P in aggregate order: 18 planes over the slots of avert
     DBuf<unsigned long long> key0, key1;
     DBuf<unsigned> val0, val1, head, hs, seg;
     DBuf<unsigned char> tmp;
     DBuf<int> info;
-    std::vector<double> hx;
-    void* handle = nullptr;  // rocblas_handle
-    CoarseWork() = default;
-    CoarseWork(const CoarseWork&) = delete;
-    CoarseWork& operator=(const CoarseWork&) = delete;
-    ~CoarseWork();
 };
 
 struct LinWork {
