@@ -382,38 +382,92 @@ __global__ void k_fill_u32(size_t n, unsigned* __restrict__ a, unsigned v)
     if (i < n) a[i] = v;
 }
 
-// Voxels of a query box split over the G lanes of a group (lane j takes the
-// linear voxel indices j, j+G, ...).  Every stored primitive of the requested
-// type whose box overlaps the query box is visited exactly once, in the
-// lowest shared voxel (componentwise max of the two box minima, clamped).
-template <int G, class F>
-__device__ inline void walk_lanes(const GridDev& g, unsigned keybase, const CellTable& T,
-                                  const int* __restrict__ pbox_t, int type, const int* ql, const int* qh, int lane,
-                                  F&& visit)
-{
-    int l[3], n[3];
-    for (int d = 0; d < 3; ++d) {
-        l[d] = max(ql[d], 0);
-        n[d] = min(qh[d], g.cnt[d] - 1) - l[d] + 1;
-        if (n[d] <= 0) return;
+// Walk of a query box by the G lanes of a group (lane j takes the linear
+// voxel indices j, j+G, ...).  Every stored primitive of the requested type
+// whose box overlaps the query box is found exactly once, in the lowest
+// shared voxel (componentwise max of the two box minima, clamped).
+template <int G>
+struct WalkLane {
+    int q[3], l[3], n[2], x, y, z;
+    unsigned nvox, li, k, e, base, sx, sy;
+    __device__ void none() { nvox = li = k = e = 0; }
+    __device__ void start(const GridDev& g, unsigned keybase, int type, const int* ql, const int* qh, int lane)
+    {
+        none();
+        unsigned m = 1;
+        int c[3];
+        for (int d = 0; d < 3; ++d) {
+            q[d] = ql[d];
+            l[d] = max(ql[d], 0);
+            c[d] = min(qh[d], g.cnt[d] - 1) - l[d] + 1;
+            if (c[d] <= 0) return;
+            m *= (unsigned)c[d];  // at most 1e9 voxels in a grid
+        }
+        n[0] = c[0];
+        n[1] = c[1];
+        base = keybase + (unsigned)type;
+        sx = (unsigned)g.cnt[0];
+        sy = (unsigned)g.cnt[1];
+        nvox = m;
+        li = (unsigned)lane;
     }
-    const long nvox = (long)n[0] * n[1] * n[2];
-    for (long li = lane; li < nvox; li += G) {
-        const int x = l[0] + (int)(li % n[0]);
-        const long r = li / n[0];
-        const int y = l[1] + (int)(r % n[1]);
-        const int z = l[2] + (int)(r / n[1]);
-        unsigned s, e;
-        cell_range(T, keybase + 2u * key_of(g, x, y, z) + (unsigned)type, s, e);
-        for (unsigned k = s; k < e; ++k) {
-            const int f = T.vals[k];
-            const int* pb = pbox_t + 6L * f;
-            if (max(max(ql[0], pb[0]), 0) != x || max(max(ql[1], pb[1]), 0) != y || max(max(ql[2], pb[2]), 0) != z)
-                continue;
-            visit(f);
+    // the next primitive found by this lane; -1 at the end
+    __device__ int next(const CellTable& T, const int* __restrict__ pbox_t)
+    {
+        for (;;) {
+            while (k < e) {
+                const int f = T.vals[k++];
+                const int* pb = pbox_t + 6L * f;
+                if (max(q[0], max(pb[0], 0)) == x && max(q[1], max(pb[1], 0)) == y && max(q[2], max(pb[2], 0)) == z)
+                    return f;
+            }
+            if (li >= nvox) return -1;
+            x = l[0] + (int)(li % (unsigned)n[0]);
+            const unsigned r = li / (unsigned)n[0];
+            y = l[1] + (int)(r % (unsigned)n[1]);
+            z = l[2] + (int)(r / (unsigned)n[1]);
+            cell_range(T, base + 2u * ((unsigned)x + sx * ((unsigned)y + sy * (unsigned)z)), k, e);
+            li += G;
         }
     }
-}
+};
+
+// Pairs (query, primitive) found by a wavefront's lanes wait in LDS until 64
+// are there, and are then tested one per lane.  Tested where they are found,
+// a few lanes at a time, the narrow phase ran with most lanes idle.
+constexpr int WALK_QUEUE = 128;
+struct WalkQueue {
+    int2* buf;  // WALK_QUEUE entries of this wavefront
+    unsigned n;
+    // called by the whole wavefront; test(pair) is called with every lane that holds one
+    template <class F>
+    __device__ void push(bool have, int2 pair, F&& test)
+    {
+        const unsigned long long m = __ballot(have);
+        const int lane = threadIdx.x & 63;
+        if (have) buf[n + (unsigned)__popcll(m & ((1ull << lane) - 1))] = pair;
+        n += (unsigned)__popcll(m);
+        __builtin_amdgcn_wave_barrier();  // a wavefront's LDS accesses are in program order
+        if (n >= 64) {
+            const int2 p = buf[lane];
+            n -= 64;
+            const int2 t = buf[64 + lane];
+            __builtin_amdgcn_wave_barrier();
+            if (lane < (int)n) buf[lane] = t;
+            __builtin_amdgcn_wave_barrier();
+            test(p, true);
+        }
+    }
+    template <class F>
+    __device__ void drain(F&& test)
+    {
+        const int lane = threadIdx.x & 63;
+        if (n == 0) return;
+        const int2 p = buf[lane];
+        test(p, lane < (int)n);
+        n = 0;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // narrow phase of the constraint set
@@ -606,40 +660,60 @@ __device__ inline void ee_narrow(const CSArgs& A, int inst, int eI, int eJ, cons
 // Constraint-set queries: q < nb are boundary vertices against triangles
 // (SPATIAL_HASH.h:215-241, box [p - r, p + r]); the rest are boundary edges
 // against edges eJ > eI (SPATIAL_HASH.h:243-291, edge box inflated by r).
-// G lanes per query.
+// G lanes per query; found pairs are tested 64 at a time.
 template <int G>
 __global__ void __launch_bounds__(256) k_cs_walk(int nb, int ne, CSArgs A, CellTable T, CSOut O)
 {
+    __shared__ int2 sh[4][WALK_QUEUE];
     const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long q = tid / G;
     const int lane = (int)(tid % G);
-    if (q >= (long)nb + ne) return;
-    int ql[3], qh[3];
-    if (q < nb) {
-        const int vI = A.bn[q];
-        const int inst = A.vinst[vI];
-        if (A.active && !A.active[inst]) return;
-        const GridDev& g = A.grids[inst];
-        const double r = A.rad[inst];
-        const d3 p = ld3(A.X, vI);
-        locate(g, p.x - r, p.y - r, p.z - r, ql);
-        locate(g, p.x + r, p.y + r, p.z + r, qh);
-        walk_lanes<G>(g, A.keybase[inst], T, A.pbox, 0, ql, qh, lane,
-                      [&](int f) { pt_narrow(A, inst, vI, f, O); });
-    } else {
-        const int eI = (int)(q - nb);
-        const int2 e = A.be[eI];
-        const int inst = A.vinst[e.x];
-        if (A.active && !A.active[inst]) return;
-        const GridDev& g = A.grids[inst];
-        const double r = A.rad[inst];
-        const d3 a = ld3(A.X, e.x), b = ld3(A.X, e.y);
-        locate(g, fmin(a.x, b.x) - r, fmin(a.y, b.y) - r, fmin(a.z, b.z) - r, ql);
-        locate(g, fmax(a.x, b.x) + r, fmax(a.y, b.y) + r, fmax(a.z, b.z) + r, qh);
-        walk_lanes<G>(g, A.keybase[inst], T, A.pbox + 6L * A.nf, 1, ql, qh, lane, [&](int f) {
-            if (f > eI) ee_narrow(A, inst, eI, f, O);
-        });
+    WalkLane<G> W;
+    W.none();
+    int eI = -1;  // edge queries take edges of larger index only
+    const int* pbox = A.pbox;
+    if (q < (long)nb + ne) {
+        int ql[3], qh[3], inst, type = 0;
+        double r;
+        if (q < nb) {
+            const int vI = A.bn[q];
+            inst = A.vinst[vI];
+            r = A.rad[inst];
+            const GridDev& g = A.grids[inst];
+            const d3 p = ld3(A.X, vI);
+            locate(g, p.x - r, p.y - r, p.z - r, ql);
+            locate(g, p.x + r, p.y + r, p.z + r, qh);
+        } else {
+            eI = (int)(q - nb);
+            const int2 e = A.be[eI];
+            inst = A.vinst[e.x];
+            r = A.rad[inst];
+            const GridDev& g = A.grids[inst];
+            const d3 a = ld3(A.X, e.x), b = ld3(A.X, e.y);
+            locate(g, fmin(a.x, b.x) - r, fmin(a.y, b.y) - r, fmin(a.z, b.z) - r, ql);
+            locate(g, fmax(a.x, b.x) + r, fmax(a.y, b.y) + r, fmax(a.z, b.z) + r, qh);
+            type = 1;
+            pbox = A.pbox + 6L * A.nf;
+        }
+        if (!(A.active && !A.active[inst])) W.start(A.grids[inst], A.keybase[inst], type, ql, qh, lane);
     }
+    WalkQueue Q{sh[threadIdx.x >> 6], 0u};
+    auto test = [&](int2 p, bool in) {
+        if (!in) return;
+        if (p.x < nb) {
+            const int vI = A.bn[p.x];
+            pt_narrow(A, A.vinst[vI], vI, p.y, O);
+        } else {
+            const int e = p.x - nb;
+            ee_narrow(A, A.vinst[A.be[e].x], e, p.y, O);
+        }
+    };
+    for (;;) {
+        const int f = W.next(T, pbox);
+        if (__ballot(f >= 0) == 0) break;
+        Q.push(f > eI, make_int2((int)q, f), test);
+    }
+    Q.drain(test);
 }
 
 // ---------------------------------------------------------------------------
@@ -732,78 +806,80 @@ __device__ inline long walk_nvox(const GridDev& g, const int* ql, const int* qh)
 }
 
 // Swept-box candidates of the CCD (SPATIAL_HASH.h:484-690): G lanes per
-// query.  BIG: the first pass (BIG = false) hands every query whose box
-// covers more than WALK_BIG_VOX voxels to a list that the second pass walks
-// with a whole workgroup per query, so one fast-moving primitive does not
-// hold the launch up on eight lanes.
-template <int G, bool BIG>
-__device__ inline void ccd_walk_query(long q, int lane, int nb, const CCDArgs& A, const CellTable& T,
-                                      unsigned* __restrict__ cnt, int2* __restrict__ cand, unsigned cap,
-                                      unsigned* __restrict__ nbig, unsigned* __restrict__ big)
-{
-    if (q < nb) {
-        const int v = A.bn[q];
-        const int inst = A.vinst[v];
-        if (A.active && !A.active[inst]) return;
-        const GridDev& g = A.grids[inst];
-        if (!BIG && walk_nvox(g, A.vbox + 6 * q, A.vbox + 6 * q + 3) > WALK_BIG_VOX) {
-            if (lane == 0) big[atomicAdd(nbig, 1u)] = (unsigned)q;
-            return;
-        }
-        const d3 p = ld3(A.X, v), dp = ld3(A.P, v);
-        walk_lanes<G>(g, A.keybase[inst], T, A.pbox, 0, A.vbox + 6 * q, A.vbox + 6 * q + 3, lane, [&](int f) {
-            const int3 t = A.bt[f];
-            const bool ok = !(v == t.x || v == t.y || v == t.z) &&
-                            !(A.dbc[v] && A.dbc[t.x] && A.dbc[t.y] && A.dbc[t.z]) &&
-                            pt_ccd_broadphase(p, ld3(A.X, t.x), ld3(A.X, t.y), ld3(A.X, t.z), dp, ld3(A.P, t.x),
-                                              ld3(A.P, t.y), ld3(A.P, t.z), A.th);
-            const unsigned i = wave_append(cnt, ok);
-            if (ok && i < cap) cand[i] = make_int2(v, f);  // PT from the front
-        });
-    } else {
-        const int eI = (int)(q - nb);
-        const int2 a = A.be[eI];
-        const int inst = A.vinst[a.x];
-        if (A.active && !A.active[inst]) return;
-        const GridDev& g = A.grids[inst];
-        const int* pe = A.pbox + 6L * A.nf;
-        const int* eb = pe + 6L * eI;
-        if (!BIG && walk_nvox(g, eb, eb + 3) > WALK_BIG_VOX) {
-            if (lane == 0) big[atomicAdd(nbig, 1u)] = (unsigned)q;
-            return;
-        }
-        const d3 a0 = ld3(A.X, a.x), a1 = ld3(A.X, a.y), da0 = ld3(A.P, a.x), da1 = ld3(A.P, a.y);
-        walk_lanes<G>(g, A.keybase[inst], T, pe, 1, eb, eb + 3, lane, [&](int f) {
-            bool ok = f > eI;
-            if (ok) {
-                const int2 b = A.be[f];
-                ok = !(a.x == b.x || a.x == b.y || a.y == b.x || a.y == b.y) &&
-                     !(A.dbc[a.x] && A.dbc[a.y] && A.dbc[b.x] && A.dbc[b.y]) &&
-                     ee_ccd_broadphase(a0, a1, ld3(A.X, b.x), ld3(A.X, b.y), da0, da1, ld3(A.P, b.x),
-                                       ld3(A.P, b.y), A.th);
-            }
-            const unsigned i = wave_append(cnt + 1, ok);
-            if (ok && i < cap) cand[cap - 1 - i] = make_int2(-eI - 1, f);  // EE from the back
-        });
-    }
-}
-
+// query, found pairs tested 64 at a time.  BIG: the first pass (BIG = false)
+// hands every query whose box covers more than WALK_BIG_VOX voxels to a list
+// that the second pass walks with a whole workgroup per query, so one
+// fast-moving primitive does not hold the launch up on a few lanes.
 template <int G, bool BIG>
 __global__ void __launch_bounds__(256) k_ccd_walk(int nb, int ne, CCDArgs A, CellTable T,
                                                   unsigned* __restrict__ cnt, int2* __restrict__ cand, unsigned cap,
                                                   unsigned* __restrict__ nbig, unsigned* __restrict__ big)
 {
+    __shared__ int2 sh[4][WALK_QUEUE];
+    const int* pe = A.pbox + 6L * A.nf;
+    WalkQueue Q{sh[threadIdx.x >> 6], 0u};
+    auto test = [&](int2 p, bool in) {
+        // all pairs of a wavefront come from few queries: mostly one kind at a time
+        bool ok = false;
+        const bool pt = in && p.x < nb;
+        if (pt) {
+            const int v = A.bn[p.x];
+            const int3 t = A.bt[p.y];
+            ok = !(v == t.x || v == t.y || v == t.z) && !(A.dbc[v] && A.dbc[t.x] && A.dbc[t.y] && A.dbc[t.z]) &&
+                 pt_ccd_broadphase(ld3(A.X, v), ld3(A.X, t.x), ld3(A.X, t.y), ld3(A.X, t.z), ld3(A.P, v),
+                                   ld3(A.P, t.x), ld3(A.P, t.y), ld3(A.P, t.z), A.th);
+            p.x = v;
+        } else if (in) {
+            const int eI = p.x - nb;
+            const int2 a = A.be[eI], b = A.be[p.y];
+            ok = !(a.x == b.x || a.x == b.y || a.y == b.x || a.y == b.y) &&
+                 !(A.dbc[a.x] && A.dbc[a.y] && A.dbc[b.x] && A.dbc[b.y]) &&
+                 ee_ccd_broadphase(ld3(A.X, a.x), ld3(A.X, a.y), ld3(A.X, b.x), ld3(A.X, b.y), ld3(A.P, a.x),
+                                   ld3(A.P, a.y), ld3(A.P, b.x), ld3(A.P, b.y), A.th);
+            p.x = -eI - 1;
+        }
+        const unsigned i = wave_append(cnt, ok && pt);
+        if (ok && pt && i < cap) cand[i] = p;  // PT from the front
+        const unsigned j = wave_append(cnt + 1, ok && !pt);
+        if (ok && !pt && j < cap) cand[cap - 1 - j] = p;  // EE from the back
+    };
+    auto walk = [&](long q, int lane) {
+        WalkLane<G> W;
+        W.none();
+        int eI = -1;  // edge queries take edges of larger index only
+        const int* pbox = A.pbox;
+        if (q >= 0) {
+            const int* box = q < nb ? A.vbox + 6 * q : pe + 6 * (q - nb);
+            const int inst = A.vinst[q < nb ? A.bn[q] : A.be[q - nb].x];
+            if (q >= nb) {
+                eI = (int)(q - nb);
+                pbox = pe;
+            }
+            if (!(A.active && !A.active[inst])) {
+                const GridDev& g = A.grids[inst];
+                if (!BIG && walk_nvox(g, box, box + 3) > WALK_BIG_VOX) {
+                    if (lane == 0) big[atomicAdd(nbig, 1u)] = (unsigned)q;
+                } else {
+                    W.start(g, A.keybase[inst], q < nb ? 0 : 1, box, box + 3, lane);
+                }
+            }
+        }
+        for (;;) {
+            const int f = W.next(T, pbox);
+            if (__ballot(f >= 0) == 0) break;
+            Q.push(f > eI, make_int2((int)q, f), test);
+        }
+    };
     if (BIG) {
         // a workgroup per listed query (the list is final: the first pass has ended)
         const unsigned n = *nbig;
-        for (unsigned k = blockIdx.x; k < n; k += gridDim.x)
-            ccd_walk_query<G, true>((long)big[k], (int)threadIdx.x, nb, A, T, cnt, cand, cap, nbig, big);
+        for (unsigned k = blockIdx.x; k < n; k += gridDim.x) walk((long)big[k], (int)threadIdx.x);
     } else {
         const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
         const long q = tid / G;
-        if (q >= (long)nb + ne) return;
-        ccd_walk_query<G, false>(q, (int)(tid % G), nb, A, T, cnt, cand, cap, nbig, big);
+        walk(q < (long)nb + ne ? q : -1, (int)(tid % G));
     }
+    Q.drain(test);
 }
 
 // ACCD over the candidates as a work queue (amin: running minimum per instance).  Each lane carries one pair
@@ -1240,7 +1316,12 @@ __global__ void k_place_merged(unsigned n, const int4* __restrict__ t, const int
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr int WALK_G = 8;                        // lanes per query
+// Lanes per query of the walks.  The voxels of a query are a chain of
+// dependent loads per lane, so few queries are spread over more lanes while
+// that fills the chip (256 CUs hold 524,288 lanes).  CCD, 17,400 queries:
+// 2.59, 1.84, 1.42, 1.00 ms with 8, 16, 32, 64 lanes; 80,000 queries (24
+// cubes): 30.6, 29.9, 30.4, 33.2 ms a step.
+inline int walk_lanes_for(long nq) { return nq <= 32768 ? 64 : nq <= 65536 ? 32 : 16; }
 constexpr unsigned long long DENSE_MAX = 1ull << 25;  // max record keys of a dense cell table
 
 unsigned read_u(hipStream_t s, const unsigned* p)
@@ -1258,7 +1339,7 @@ int bits_for(unsigned long long maxv)
     return b;
 }
 
-int walk_blocks(long nq) { return grid_for(nq * WALK_G, 256); }
+int walk_blocks(long nq, int g) { return grid_for(nq * g, 256); }
 
 // Boxes of the triangles and edges from the vertex boxes, their sorted
 // (keybase[instance] + 2 * voxel + type, primitive) records and the cell
@@ -1411,7 +1492,12 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
             O.cap_p = (unsigned)std::min(w.pk0.cap, w.pass.cap);
             O.cap_d = (unsigned)w.dk0.cap;
             IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, cnt, 2);
-            IDP_LAUNCH(k_cs_walk<WALK_G>, walk_blocks((long)m.nb + m.ne), 256, 0, s, m.nb, m.ne, A, T, O);
+            // the boxes of static queries are small: half of the CCD's lanes each
+            const int G = walk_lanes_for((long)m.nb + m.ne) / 2;
+            const int wb = walk_blocks((long)m.nb + m.ne, G);
+            if (G == 32) IDP_LAUNCH(k_cs_walk<32>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
+            else if (G == 16) IDP_LAUNCH(k_cs_walk<16>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
+            else IDP_LAUNCH(k_cs_walk<8>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
             IDP_HIP(hipMemcpyAsync(hc, cnt, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, s));
             IDP_HIP(hipStreamSynchronize(s));
             if (hc[0] <= O.cap_p && hc[1] <= O.cap_d) break;
@@ -1583,8 +1669,13 @@ void contact_ccd_batch(ContactWork& w, hipStream_t s, const MeshDev& m, const do
             unsigned* nbig = cnt + 5;
             unsigned* big = w.walk_big.ensure((size_t)m.nb + m.ne + 1, s);
             IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, nbig, 1);
-            IDP_LAUNCH((k_ccd_walk<WALK_G, false>), walk_blocks((long)m.nb + m.ne), 256, 0, s, m.nb, m.ne, A, T,
-                       cnt, cand, cap, nbig, big);
+            const int G = walk_lanes_for((long)m.nb + m.ne), wb = walk_blocks((long)m.nb + m.ne, G);
+            if (G == 64)
+                IDP_LAUNCH((k_ccd_walk<64, false>), wb, 256, 0, s, m.nb, m.ne, A, T, cnt, cand, cap, nbig, big);
+            else if (G == 32)
+                IDP_LAUNCH((k_ccd_walk<32, false>), wb, 256, 0, s, m.nb, m.ne, A, T, cnt, cand, cap, nbig, big);
+            else
+                IDP_LAUNCH((k_ccd_walk<16, false>), wb, 256, 0, s, m.nb, m.ne, A, T, cnt, cand, cap, nbig, big);
             // large queries: one workgroup each
             IDP_LAUNCH((k_ccd_walk<256, true>), (int)std::min<long>((long)m.nb + m.ne, 2048), 256, 0, s, m.nb,
                        m.ne, A, T, cnt, cand, cap, nbig, big);
