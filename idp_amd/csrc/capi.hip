@@ -104,6 +104,7 @@ struct idp_ctx {
     // entry points (resolved once per device when the first context is created)
     unsigned char* scratch = nullptr;
     FricState fr;
+    PinBuf pin;  // results read back
 };
 
 namespace {
@@ -315,6 +316,16 @@ void friction_basis(idp_ctx* c, const double* X, double dHat2, double kappa, dou
     f.have = true;
 }
 
+// a device byte holding 1: the warm-start mask of a one-mesh solve
+const unsigned char* one_byte(idp_ctx* c)
+{
+    if (!c->one.p) {
+        static const unsigned char on = 1;
+        c->one.upload(&on, 1, c->s);
+    }
+    return c->one.p;
+}
+
 // the contact BSR structure of the current constraint set, followed by the
 // friction set while friction is on
 void build_contact_structure(idp_ctx* c)
@@ -324,9 +335,34 @@ void build_contact_structure(idp_ctx* c)
                       fo ? (const int*)c->fr.fcs.p : nullptr);
 }
 
+// block table of n elements of one instance: blocks of RB, as SegDev::build makes it
+__global__ void k_seg_one(int nblk, int n, int* __restrict__ lo, int* __restrict__ hi, int* __restrict__ inst,
+                          int* __restrict__ pbeg)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        pbeg[0] = 0;
+        pbeg[1] = nblk;
+    }
+    if (i >= nblk) return;
+    lo[i] = RB * i;
+    hi[i] = min(RB * (i + 1), n);
+    inst[i] = 0;
+}
+
 void update_cseg(idp_ctx* c)
 {
     if (c->cw.h_cbeg.size() != (size_t)c->m.inst.B + 1) c->cw.h_cbeg = {0, c->cw.ncs};
+    if (c->m.inst.B == 1) {  // formed on the device: nothing to upload per constraint set
+        SegDev& g = c->cseg;
+        g.bs = RB;
+        g.nblk = grid_for(c->cw.ncs, RB);
+        g.h_pbeg = {0, g.nblk};
+        IDP_LAUNCH(k_seg_one, grid_for(std::max(g.nblk, 1), 256), 256, 0, c->s, g.nblk, (int)c->cw.ncs,
+                   g.lo.ensure(g.nblk, c->s), g.hi.ensure(g.nblk, c->s), g.inst.ensure(g.nblk, c->s),
+                   g.pbeg.ensure(2, c->s));
+        return;
+    }
     c->cseg.build(c->cw.h_cbeg, RB, c->s);
 }
 
@@ -349,7 +385,9 @@ void energies(idp_ctx* c, const double* X, bool with_barrier, double h, std::vec
     auto& m = c->m;
     const InstDev& I = m.inst;
     const int B = I.B;
-    int* fl = c->flags.ensure(2 * (size_t)B + 4, s);
+    // sums, then the flags: read back together
+    double* es = c->esum.ensure(7 * (size_t)B, s);
+    int* fl = (int*)(es + 6 * (size_t)B);
     IDP_HIP(hipMemsetAsync(fl, 0, 2 * B * sizeof(int), s));
     const int tok = c->prof.begin(IDP_K_ENERGY);
     double* pe = c->part_e.ensure(I.tblk.nblk + 1, s);
@@ -361,7 +399,6 @@ void energies(idp_ctx* c, const double* X, bool with_barrier, double h, std::vec
     const bool bar = with_barrier && c->cw.ncs > 0;
     const bool flow = c->no_elastic && m.nE > 0;
     const bool shell = !c->no_elastic && m.nE > 0;  // membrane + bending
-    double* es = c->esum.ensure(6 * (size_t)B, s);
     const bool fric = with_barrier && c->fr.on && c->fr.n > 0;  // single-mesh contexts only
     IDP_LAUNCH(k_seg_sums, B, RB, 0, s, I.tblk.pbeg.p, pe, es);
     IDP_LAUNCH(k_seg_sums, B, RB, 0, s, I.vblk.pbeg.p, pi, es + B);
@@ -390,15 +427,14 @@ void energies(idp_ctx* c, const double* X, bool with_barrier, double h, std::vec
         launch_sum_partials(s, nb, pf, es + 5 * B);
     }
     c->prof.end(IDP_K_ENERGY, tok);
-    std::vector<int> hf(2 * B);
-    std::vector<double> he(6 * B, 0.0);
-    IDP_HIP(hipMemcpyAsync(hf.data(), fl, 2 * B * sizeof(int), hipMemcpyDeviceToHost, s));
-    IDP_HIP(hipMemcpyAsync(he.data(), es, (bar ? 3 : 2) * B * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (flow || shell)
-        IDP_HIP(hipMemcpyAsync(he.data() + 3 * B, es + 3 * B, (shell ? 2 : 1) * B * sizeof(double),
-                               hipMemcpyDeviceToHost, s));
-    if (fric) IDP_HIP(hipMemcpyAsync(he.data() + 5 * B, es + 5 * B, sizeof(double), hipMemcpyDeviceToHost, s));
+    double* he = c->pin.as<double>(7 * (size_t)B);
+    IDP_HIP(hipMemcpyAsync(he, es, 7 * (size_t)B * sizeof(double), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
+    const int* hf = (const int*)(he + 6 * (size_t)B);
+    for (int i = 0; i < B; ++i) {  // the terms that were not formed
+        if (!flow && !shell) he[3 * B + i] = 0.0;
+        if (!shell) he[4 * B + i] = 0.0;
+    }
     out.resize(B);
     for (int i = 0; i < B; ++i) {
         EnergyOut& o = out[i];
@@ -417,20 +453,19 @@ EnergyOut energy(idp_ctx* c, const double* X, bool with_barrier, double h)
     return o[0];
 }
 
+__global__ void k_set_u64(unsigned long long* __restrict__ p, unsigned long long v) { *p = v; }
+
 double min_dist2_dev(idp_ctx* c, const double* X, long n, const int* cs, double* dist2)
 {
     IDP_TIMER_FLAG("Compute_Min_Dist");
     auto s = c->s;
     unsigned long long* dm = c->dmin.ensure(1, s);
-    unsigned long long init = 0x7ff0000000000000ull;  // +inf
-    IDP_HIP(hipMemcpyAsync(dm, &init, sizeof(init), hipMemcpyHostToDevice, s));
+    IDP_LAUNCH(k_set_u64, 1, 1, 0, s, dm, 0x7ff0000000000000ull);  // +inf
     launch_min_dist2(s, n, cs, X, nullptr, dist2, dm);
-    unsigned long long r;
-    IDP_HIP(hipMemcpyAsync(&r, dm, sizeof(r), hipMemcpyDeviceToHost, s));
+    double* r = c->pin.as<double>(1);
+    IDP_HIP(hipMemcpyAsync(r, dm, sizeof(double), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
-    double d;
-    std::memcpy(&d, &r, sizeof(d));
-    return d;
+    return *r;
 }
 
 // gradient at X with the current constraint set (structure must be built);
@@ -2218,8 +2253,7 @@ int idp_advance_one_step(idp_ctx* c, double h, double newton_tol, int with_colli
                 t0 = now_ms();
                 double rel = 0;
                 // from the second Newton iteration on, sol holds this step's previous direction
-                const unsigned char on = 1;
-                const unsigned char* warm = PNIter > 0 && !cold ? c->one.upload_get(&on, 1, s) : nullptr;
+                const unsigned char* warm = PNIter > 0 && !cold ? one_byte(c) : nullptr;
                 int it;
                 {
                     IDP_TIMER_FLAG("linearSolve");
@@ -2315,16 +2349,14 @@ int idp_advance_one_step(idp_ctx* c, double h, double newton_tol, int with_colli
                 long np = c->ncs_prev;
                 double* cur = c->tmpv.ensure(np, s);
                 min_dist2_dev(c, x, np, (const int*)csp.p, cur);
-                std::vector<double> hc(np), hp(np);
-                IDP_HIP(hipMemcpyAsync(hc.data(), cur, np * 8, hipMemcpyDeviceToHost, s));
-                IDP_HIP(hipMemcpyAsync(hp.data(), c->dist2_prev.p, np * 8, hipMemcpyDeviceToHost, s));
+                int* kflag = c->flags.ensure(4, s);
+                IDP_HIP(hipMemsetAsync(kflag, 0, sizeof(int), s));
+                IDP_LAUNCH(k_kappa_test, grid_for(np, 256), 256, 0, s, np, csp.p, m.inst.vinst.p, cur, c->dist2_prev.p,
+                           kflag);
+                int* hk = c->pin.as<int>(1);
+                IDP_HIP(hipMemcpyAsync(hk, kflag, sizeof(int), hipMemcpyDeviceToHost, s));
                 IDP_HIP(hipStreamSynchronize(s));
-                bool upd = false;
-                for (long i = 0; i < np; ++i)
-                    if (hp[i] < 1e-18 && hc[i] < hp[i]) {
-                        upd = true;
-                        break;
-                    }
+                const bool upd = *hk != 0;
                 if (upd && kappa < kappa3[1]) {
                     kappa *= 2;
                     kappa3[0] = kappa;
@@ -2385,12 +2417,11 @@ int idp_advance_one_step(idp_ctx* c, double h, double newton_tol, int with_colli
                         IDP_LAUNCH(k_dbc_hess, grid_for(nd, 256), 256, 0, s, nd, c->dbc_idx_d.p, m.mass.p, m.proj,
                                    m.e_diag.p, m.nnzb_e, DBCStiff, c->L.evals.p);
                     double rel = 0;
-                    const unsigned char on = 1;
                     int it;
                     {
                         IDP_TIMER_FLAG("linearSolve");
                         it = pcg_solve_persistent(c->L, s, m, rhs, sol, rtol, maxit, &rel,
-                                                  cold ? nullptr : c->one.upload_get(&on, 1, s));
+                                                  cold ? nullptr : one_byte(c));
                     }
                     if (it < 0) {  // the reference exits when this solve fails (IMPLICIT_EULER.h:818-825)
                         c->err = "linear solve failed after a friction basis update";

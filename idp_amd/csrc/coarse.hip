@@ -661,8 +661,8 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
     const int nbox = std::min(grid_for(nV, 256), 64);
     double* dbox = C.box.ensure(7 * (size_t)nbox, s);
     IDP_LAUNCH(k_coarse_box, nbox, 256, 0, s, nV, X, m.proj_mask(), dbox);
-    std::vector<double> hb(7 * (size_t)nbox);
-    IDP_HIP(hipMemcpyAsync(hb.data(), dbox, hb.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    double* hb = L.pin.as<double>(7 * (size_t)nbox);
+    IDP_HIP(hipMemcpyAsync(hb, dbox, 7 * (size_t)nbox * sizeof(double), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     long nfree = 0;
@@ -713,9 +713,10 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
         unsigned* dc = C.ccnt.ensure(ncell, s);
         IDP_LAUNCH(k_coarse_zero, grid_for(ncell, 256), 256, 0, s, (long)ncell, dc);
         IDP_LAUNCH(k_coarse_cells, grid_for(nV, 256), 256, 0, s, nV, X, m.proj_mask(), g, ncell, key, vert, dc);
-        cnt.resize(ncell);
-        IDP_HIP(hipMemcpyAsync(cnt.data(), dc, ncell * sizeof(unsigned), hipMemcpyDeviceToHost, s));
+        unsigned* hc = L.pin.as<unsigned>(ncell);
+        IDP_HIP(hipMemcpyAsync(hc, dc, ncell * sizeof(unsigned), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
+        cnt.assign(hc, hc + ncell);
         K = 0;
         for (unsigned q : cnt) K += q > 0;
         if (K <= COARSE_MAX_AGG) break;
@@ -798,10 +799,10 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
                    D + ((k + 1) & 1) * SW * SW, info);
         std::swap(src, dst);
     }
-    int hinfo = 0;
-    IDP_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s));
+    int* hinfo = L.pin.as<int>(1);
+    IDP_HIP(hipMemcpyAsync(hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
-    if (hinfo != 0) return false;  // not positive definite: no coarse level this time
+    if (*hinfo != 0) return false;  // not positive definite: no coarse level this time
     C.rc.ensure(ncd, s);
     C.nsb = K;  // one partial of r_c . e_c per aggregate
     C.part.ensure(2 * (size_t)C.nsb + 2, s);

@@ -136,6 +136,36 @@ struct DBuf {
     }
 };
 
+// Page-locked host memory that small results are read back into: a copy to
+// pageable memory stops the host once per copy (10-25 us), these are queued
+// together and waited for once.
+struct PinBuf {
+    void* p = nullptr;
+    size_t cap = 0;
+    PinBuf() = default;
+    PinBuf(const PinBuf&) = delete;
+    PinBuf& operator=(const PinBuf&) = delete;
+    ~PinBuf()
+    {
+        if (p) (void)hipHostFree(p);
+    }
+    // contents are lost when it grows
+    template <class T>
+    T* as(size_t n)
+    {
+        const size_t bytes = n * sizeof(T);
+        if (bytes > cap) {
+            void* q = nullptr;
+            const size_t nc = std::max<size_t>(bytes + bytes / 2, 4096);
+            IDP_HIP(hipHostMalloc(&q, nc));
+            if (p) (void)hipHostFree(p);
+            p = q;
+            cap = nc;
+        }
+        return (T*)p;
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Optional per-family device timing with HIP events on one stream.  Records
 // stay open until collect(); a caller may discard records it tagged (e.g. the

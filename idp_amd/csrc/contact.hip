@@ -1236,7 +1236,7 @@ __global__ void __launch_bounds__(256) k_accd(const unsigned* __restrict__ cnt, 
 // instance's ACCD bound
 __global__ void k_ccd_cap(int B, const double* __restrict__ eparts, const int* __restrict__ epbeg,
                           const int* __restrict__ ebeg, const double* __restrict__ psum, const int* __restrict__ nbeg,
-                          const double* __restrict__ alpha_in, double* __restrict__ alpha_out,
+                          const double* __restrict__ alpha_in, double alpha1, double* __restrict__ alpha_out,
                           unsigned long long* __restrict__ amin, const unsigned char* __restrict__ active)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1246,7 +1246,7 @@ __global__ void k_ccd_cap(int B, const double* __restrict__ eparts, const int* _
     const long ne = ebeg[i + 1] - ebeg[i], nb = nbeg[i + 1] - nbeg[i];
     vs = ne ? vs / (double)ne : 1.0;
     ps = psum[i] / (double)(nb * 3);
-    double a = alpha_in[i];
+    double a = alpha_in ? alpha_in[i] : alpha1;
     const double span = a * ps / vs;
     if (span > 1) a /= span;
     alpha_out[i] = a;
@@ -1260,15 +1260,17 @@ __global__ void k_reset_amin(int B, const double* __restrict__ alpha, unsigned l
     if (i < B && (!active || active[i])) amin[i] = (unsigned long long)__double_as_longlong(alpha[i]);
 }
 
-__global__ void k_zero_u64(unsigned long long* __restrict__ a, int n)
-{
-    if ((int)threadIdx.x < n) a[threadIdx.x] = 0ull;
-}
-
-__global__ void k_zero_u8(unsigned char* __restrict__ a, int n)
+// counters of a CCD call: queue, statistics, per-instance hand-over marks and cap counts
+__global__ void k_ccd_zero(int B, unsigned* __restrict__ cnt, unsigned long long* __restrict__ stepstat,
+                           unsigned char* __restrict__ pend, unsigned* __restrict__ capcnt)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = 0;
+    if (i < 6) cnt[i] = 0u;
+    if (i < 4) stepstat[i] = 0ull;
+    if (i < B) {
+        pend[i] = 0;
+        capcnt[i] = 0u;
+    }
 }
 
 __global__ void k_zero_u32(unsigned* __restrict__ a, int n)
@@ -1324,12 +1326,12 @@ namespace {
 inline int walk_lanes_for(long nq) { return nq <= 32768 ? 64 : nq <= 65536 ? 32 : 16; }
 constexpr unsigned long long DENSE_MAX = 1ull << 25;  // max record keys of a dense cell table
 
-unsigned read_u(hipStream_t s, const unsigned* p)
+unsigned read_u(PinBuf& pin, hipStream_t s, const unsigned* p)
 {
-    unsigned v;
-    IDP_HIP(hipMemcpyAsync(&v, p, sizeof(v), hipMemcpyDeviceToHost, s));
+    unsigned* v = pin.as<unsigned>(1);
+    IDP_HIP(hipMemcpyAsync(v, p, sizeof(unsigned), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
-    return v;
+    return *v;
 }
 
 int bits_for(unsigned long long maxv)
@@ -1360,11 +1362,12 @@ CellTable build_cells(ContactWork& w, hipStream_t s, const MeshDev& m, const int
                w.grids.p, pbox + 6 * (size_t)m.nf, cnt + m.nf, pinst + m.nf);
     IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, cnt + n, 1);
     excl_scan(s, w.tmp, cnt, off, n + 1);
-    unsigned total = 0;
-    std::vector<GridDev> hg(B);
-    IDP_HIP(hipMemcpyAsync(&total, off + n, sizeof(unsigned), hipMemcpyDeviceToHost, s));
-    IDP_HIP(hipMemcpyAsync(hg.data(), w.grids.p, B * sizeof(GridDev), hipMemcpyDeviceToHost, s));
+    GridDev* hg = w.pin.as<GridDev>(B + 1);
+    unsigned* htotal = (unsigned*)(hg + B);
+    IDP_HIP(hipMemcpyAsync(htotal, off + n, sizeof(unsigned), hipMemcpyDeviceToHost, s));
+    IDP_HIP(hipMemcpyAsync(hg, w.grids.p, B * sizeof(GridDev), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
+    const unsigned total = *htotal;
     CellTable T{};
     T.n = total;
     // key bases: instance i owns keys [base_i, base_i + 2 * voxels_i)
@@ -1376,7 +1379,11 @@ CellTable build_cells(ContactWork& w, hipStream_t s, const MeshDev& m, const int
         if (acc >= 0xFFFFFFFFull) throw HipError(IDP_E_CAPACITY, "voxel key space exceeds 32 bits");
     }
     base[B] = (unsigned)acc;
-    w.keybase.upload(base.data(), B + 1, s);
+    // (an instance's end is not read on the device, so one instance's is always {0, ..})
+    if (w.h_keybase.size() != (size_t)B + 1 || !std::equal(base.begin(), base.end() - 1, w.h_keybase.begin())) {
+        w.keybase.upload(base.data(), B + 1, s);
+        w.h_keybase = base;
+    }
     if (total == 0) return T;
     unsigned* k0 = w.k0.ensure(total, s);
     int* v0 = w.v0.ensure(total, s);
@@ -1471,7 +1478,11 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
     A.keybase = w.keybase.p;
     A.vinst = I.vinst.p;
     A.active = active;
-    A.rad = w.rad.upload_get(rad.data(), rad.size(), s);
+    if (rad != w.h_rad) {
+        w.rad.upload(rad.data(), rad.size(), s);
+        w.h_rad = rad;
+    }
+    A.rad = w.rad.p;
     A.B = B;
     A.nf = m.nf;
     CSOut O;
@@ -1498,8 +1509,11 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
             if (G == 32) IDP_LAUNCH(k_cs_walk<32>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
             else if (G == 16) IDP_LAUNCH(k_cs_walk<16>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
             else IDP_LAUNCH(k_cs_walk<8>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
-            IDP_HIP(hipMemcpyAsync(hc, cnt, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, s));
+            unsigned* h = w.pin.as<unsigned>(2);
+            IDP_HIP(hipMemcpyAsync(h, cnt, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, s));
             IDP_HIP(hipStreamSynchronize(s));
+            hc[0] = h[0];
+            hc[1] = h[1];
             if (hc[0] <= O.cap_p && hc[1] <= O.cap_d) break;
             w.cap_pass = std::max<size_t>(w.cap_pass, hc[0] + hc[0] / 4 + 1024);
             w.cap_dup = std::max<size_t>(w.cap_dup, hc[1] + hc[1] / 4 + 1024);
@@ -1508,10 +1522,13 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
         clear_cells(w, s, T);
     }
     const unsigned npass = hc[0], nd = hc[1];
+    // one mesh: [pass | merged] are formed in place
+    const bool direct = B == 1 && !active;
+    if (direct) w.cs.ensure((size_t)npass + nd + 1, s);
     // ---- order the pass tuples
     if (npass) {
         unsigned long long* pk1 = w.pk1.ensure(npass, s);
-        int4* pv1 = w.dup.ensure(npass, s);
+        int4* pv1 = direct ? w.cs.p : w.dup.ensure(npass, s);
         sort_pairs(s, w.tmp, w.pk0.p, pk1, w.pass.p, pv1, npass, bits_for(((unsigned long long)B << 40) | (1ull << 40)));
     }
     // ---- merge duplicates (IPC.h:599-654)
@@ -1524,20 +1541,14 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
         IDP_LAUNCH(k_dup_heads, grid_for(nd, 256), 256, 0, s, nd, k1, head);
         IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, head + nd, 1);
         excl_scan(s, w.tmp, head, hs, nd + 1);
-        nmerged = read_u(s, hs + nd);
-        w.merged.ensure(nmerged + 1, s);
-        IDP_LAUNCH(k_dup_write, grid_for(nd, 256), 256, 0, s, nd, k1, hs, I.d_vbeg.p, O.inst_shift, w.merged.p);
+        nmerged = read_u(w.pin, s, hs + nd);
+        int4* mout = direct ? w.cs.p + npass : w.merged.ensure(nmerged + 1, s);
+        IDP_LAUNCH(k_dup_write, grid_for(nd, 256), 256, 0, s, nd, k1, hs, I.d_vbeg.p, O.inst_shift, mout);
     }
-    if (B == 1 && !active) {
-        const long total = (long)npass + nmerged;
-        int4* cs = w.cs.ensure(total + 1, s);
-        if (npass) IDP_HIP(hipMemcpyAsync(cs, w.dup.p, sizeof(int4) * npass, hipMemcpyDeviceToDevice, s));
-        if (nmerged)
-            IDP_HIP(hipMemcpyAsync(cs + npass, w.merged.p, sizeof(int4) * nmerged, hipMemcpyDeviceToDevice, s));
-        w.ncs = total;
-        w.h_cbeg = {0, total};
-        w.cbeg.upload(w.h_cbeg.data(), 2, s);
-        return total;
+    if (direct) {
+        w.ncs = (long)npass + nmerged;
+        w.h_cbeg = {0, w.ncs};
+        return w.ncs;
     }
     // ---- several instances: [pass_i | merged_i] per instance; inactive
     // instances keep their previous constraints
@@ -1613,19 +1624,22 @@ void contact_ccd_batch(ContactWork& w, hipStream_t s, const MeshDev& m, const do
     double* pp = ep + I.echunk.nblk + 1;
     IDP_LAUNCH(k_edge_len_parts, I.echunk.nblk, 256, 0, s, I.echunk.lo.p, I.echunk.hi.p, (const int2*)m.be.p, X, ep);
     IDP_LAUNCH(k_psize_seq, B, 256, 0, s, B, I.d_nbeg.p, m.bn.p, P, pp, active);
-    double* ain = (double*)w.scal2.ensure(2 * (size_t)B + 4, s);
-    IDP_HIP(hipMemcpyAsync(ain, alpha_io, B * sizeof(double), hipMemcpyHostToDevice, s));
+    const double* ain = nullptr;  // one instance: a kernel argument
+    if (B > 1) {
+        double* d = w.scal2.ensure(2 * (size_t)B + 4, s);
+        IDP_HIP(hipMemcpyAsync(d, alpha_io, B * sizeof(double), hipMemcpyHostToDevice, s));
+        ain = d;
+    }
     double* dalpha = w.ialpha.ensure(B, s);
-    unsigned long long* amin = w.iamin.ensure(B, s);
-    unsigned* cnt = w.cnt.ensure(6, s);
-    unsigned long long* stepstat = (unsigned long long*)w.scal.ensure(6, s) + 2;  // total, max, capped, certified
-    IDP_LAUNCH(k_ccd_cap, grid_for(B, 64), 64, 0, s, B, ep, I.echunk.pbeg.p, I.d_ebeg.p, pp, I.d_nbeg.p, ain, dalpha,
-               amin, active);
-    IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, cnt, 6);
-    IDP_LAUNCH(k_zero_u64, 1, 64, 0, s, stepstat, 4);
-    IDP_LAUNCH(k_zero_u8, grid_for(B, 256), 256, 0, s, pend, B);
+    // running minima, statistics (total, max, capped, certified) and counters in one piece: read back together
+    unsigned long long* amin = w.iamin.ensure((size_t)B + 7, s);
+    unsigned long long* stepstat = amin + B;
+    unsigned* cnt = (unsigned*)(stepstat + 4);
+    IDP_LAUNCH(k_ccd_cap, grid_for(B, 64), 64, 0, s, B, ep, I.echunk.pbeg.p, I.d_ebeg.p, pp, I.d_nbeg.p, ain,
+               alpha_io[0], dalpha, amin, active);
     unsigned* capcnt = w.icap.ensure(B, s);
-    IDP_LAUNCH(k_fill_u32, grid_for(B, 256), 256, 0, s, (size_t)B, capcnt, 0u);
+    const int zb = grid_for(std::max(B, 6), 256);
+    IDP_LAUNCH(k_ccd_zero, zb, 256, 0, s, B, cnt, stepstat, pend, capcnt);
     double* lg = w.accd_log.ensure(ACCD_LOG_W * ACCD_LOG_MAX, s);
 
     // swept grid over boundary nodes at [x, x + alpha p] -/+ th/2 (SPATIAL_HASH.h:484-511)
@@ -1660,15 +1674,11 @@ void contact_ccd_batch(ContactWork& w, hipStream_t s, const MeshDev& m, const do
         const unsigned cap = (unsigned)w.cand.cap;
         if (attempt) {
             IDP_LAUNCH(k_reset_amin, grid_for(B, 64), 64, 0, s, B, dalpha, amin, active);
-            IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, cnt, 6);
-            IDP_LAUNCH(k_zero_u64, 1, 64, 0, s, stepstat, 4);
-            IDP_LAUNCH(k_zero_u8, grid_for(B, 256), 256, 0, s, pend, B);
-            IDP_LAUNCH(k_fill_u32, grid_for(B, 256), 256, 0, s, (size_t)B, capcnt, 0u);
+            IDP_LAUNCH(k_ccd_zero, zb, 256, 0, s, B, cnt, stepstat, pend, capcnt);
         }
         if (T.n) {
             unsigned* nbig = cnt + 5;
             unsigned* big = w.walk_big.ensure((size_t)m.nb + m.ne + 1, s);
-            IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, nbig, 1);
             const int G = walk_lanes_for((long)m.nb + m.ne), wb = walk_blocks((long)m.nb + m.ne, G);
             if (G == 64)
                 IDP_LAUNCH((k_ccd_walk<64, false>), wb, 256, 0, s, m.nb, m.ne, A, T, cnt, cand, cap, nbig, big);
@@ -1706,10 +1716,12 @@ void contact_ccd_batch(ContactWork& w, hipStream_t s, const MeshDev& m, const do
             IDP_HIP(hipEventDestroy(e0));
             IDP_HIP(hipEventDestroy(e1));
         }
-        IDP_HIP(hipMemcpyAsync(ha.data(), amin, B * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-        IDP_HIP(hipMemcpyAsync(hsteps, stepstat, sizeof(hsteps), hipMemcpyDeviceToHost, s));
-        IDP_HIP(hipMemcpyAsync(hn, cnt, sizeof(hn), hipMemcpyDeviceToHost, s));
+        unsigned long long* h = w.pin.as<unsigned long long>((size_t)B + 7);
+        IDP_HIP(hipMemcpyAsync(h, amin, ((size_t)B + 7) * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
+        std::copy(h, h + B, ha.begin());
+        std::copy(h + B, h + B + 4, hsteps);
+        std::memcpy(hn, h + B + 4, sizeof(hn));
         const size_t total = (size_t)hn[0] + hn[1];
         if (total <= cap) break;
         w.cap_cand = std::max<size_t>(w.cap_cand, total + total / 4 + 4096);

@@ -165,6 +165,9 @@ struct ContactWork {
     bool accd_cert = true;    // long ACCD pairs try the no-hit certificate
     std::vector<unsigned> h_capped;  // ... per instance
     DBuf<unsigned> icap;
+    PinBuf pin;                        // results read back
+    std::vector<double> h_rad;         // what rad and keybase hold
+    std::vector<unsigned> h_keybase;
     Profiler* prof = nullptr;
 };
 

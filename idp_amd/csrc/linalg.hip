@@ -142,11 +142,13 @@ __global__ void k_run_heads(unsigned n, const unsigned long long* __restrict__ k
 }
 
 __global__ void k_contact_pattern(unsigned n, const unsigned long long* __restrict__ keys,
-                                  const unsigned* __restrict__ hs, unsigned long long V, unsigned* __restrict__ seg,
+                                  const unsigned* __restrict__ hs, unsigned long long V, unsigned nb,
+                                  unsigned* __restrict__ seg,
                                   int* __restrict__ crow, int* __restrict__ ccol, int* __restrict__ cdiag)
 {
     unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (i == 0) seg[nb] = n;
     if (!(i == 0 || keys[i] != keys[i - 1])) return;
     unsigned b = hs[i];
     seg[b] = i;
@@ -1245,6 +1247,8 @@ struct TeamArgs {
     int* ctl;         // [0] a wait ran out (the launch is void), [1] solves stopped, [2] hand-over after this many
                       // iterations (0: not yet)
     int* done;        // per instance: iterations done by this call when handed over
+    unsigned* start;  // per instance: workgroups of its team that are resident, TEAM_LEFT when one has left
+    long start_limit; // polls of the wait for all of them
     int nstart;       // hand-over: solves at launch (0: never)
     long spin_limit;  // polls of one wait at most
     // coarse level (one instance; K = 0: none)
@@ -1334,6 +1338,25 @@ __device__ inline bool team_meet(const TeamArgs& T, const unsigned long long* w,
     }
     __syncthreads();
     return ONE || *bad == 0;
+}
+
+// A team starts when all of its workgroups are resident: only then can they
+// wait for each other.  Nothing reserves the CUs (a cooperative launch would,
+// but only one process can hold that queue), so a workgroup that has waited
+// too long for the others leaves, if the team is still incomplete, and then
+// all of them do: the solve was not touched and runs in the two-kernel loop.
+constexpr unsigned TEAM_LEFT = 0x80000000u;
+__device__ inline bool team_start(unsigned* word, unsigned size, long limit)
+{
+    unsigned w = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    for (long k = 0;; ++k) {
+        if (w & TEAM_LEFT) return false;
+        if (w == size) return true;
+        if (k >= limit && __hip_atomic_compare_exchange_strong(word, &w, w | TEAM_LEFT, __ATOMIC_RELAXED,
+                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            return false;  // (on failure w is the word as it stands)
+        if (k < limit) w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 // cross-lane moves of a double within a row of 16 lanes (DPP; an LDS
@@ -1624,7 +1647,11 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
         rank = uni(t.y);
         size = uni(t.z);
     }
-    if (A.flag[inst] != 0) return;  // not solving (uniform over the team: written at a solve's end only)
+    if (!ONE && size > 1) {
+        if (tid == 0) bad = team_start(T.start + inst, (unsigned)size, T.start_limit) ? 0 : 1;
+        __syncthreads();
+        if (bad) return;
+    }
     const int v0 = uni(T.vbeg[inst]), v1 = uni(T.vbeg[inst + 1]);
     const int pb = uni(A.bpbeg[inst]), nb = uni(A.bpbeg[inst + 1]) - pb;
     const int ab = uni(A.apbeg[inst]), na = uni(A.apbeg[inst + 1]) - ab;
@@ -2003,12 +2030,12 @@ __global__ void __launch_bounds__(RB) k_dot_parts(long n, const double* __restri
 // host side
 // ---------------------------------------------------------------------------
 namespace {
-unsigned read_u(hipStream_t s, const unsigned* p)
+unsigned read_u(PinBuf& pin, hipStream_t s, const unsigned* p)
 {
-    unsigned v;
-    IDP_HIP(hipMemcpyAsync(&v, p, sizeof(v), hipMemcpyDeviceToHost, s));
+    unsigned* v = pin.as<unsigned>(1);
+    IDP_HIP(hipMemcpyAsync(v, p, sizeof(unsigned), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
-    return v;
+    return *v;
 }
 int bits_for(unsigned long long maxv)
 {
@@ -2034,7 +2061,7 @@ void contact_structure(LinWork& L, hipStream_t s, int nV, long ncs0, const int* 
     IDP_LAUNCH(k_contact_nv2, grid_for(ncs, 256), 256, 0, s, ncs, nv, cnt);
     IDP_HIP(hipMemsetAsync(cnt + ncs, 0, sizeof(unsigned), s));
     excl_scan<unsigned>(s, L.tmp, cnt, off, (int)ncs + 1);
-    unsigned nrec = read_u(s, off + ncs);
+    unsigned nrec = read_u(L.pin, s, off + ncs);
     unsigned long long V = (unsigned long long)nV;
     unsigned long long* k0 = L.key0.ensure(nrec, s);
     unsigned* v0 = L.rv0.ensure(nrec, s);
@@ -2046,20 +2073,18 @@ void contact_structure(LinWork& L, hipStream_t s, int nV, long ncs0, const int* 
     unsigned* hs = L.u1.ensure(nrec + 1, s);
     IDP_LAUNCH(k_run_heads, grid_for(nrec + 1, 256), 256, 0, s, nrec, k1, head);
     excl_scan<unsigned>(s, L.tmp, head, hs, (int)nrec + 1);
-    unsigned nb = read_u(s, hs + nrec);
+    unsigned nb = read_u(L.pin, s, hs + nrec);
     unsigned* seg = L.seg.ensure(nb + 1, s);
     int* crow = L.crow.ensure(nb + 1, s);
     int* ccol = L.ccol.ensure(nb + 1, s);
     int* cdiag = L.cdiag.ensure(nV, s);
     IDP_HIP(hipMemsetAsync(cdiag, 0xff, sizeof(int) * nV, s));
-    IDP_LAUNCH(k_contact_pattern, grid_for(nrec, 256), 256, 0, s, nrec, k1, hs, V, seg, crow, ccol, cdiag);
-    IDP_HIP(hipMemcpyAsync(seg + nb, &nrec, sizeof(unsigned), hipMemcpyHostToDevice, s));
+    IDP_LAUNCH(k_contact_pattern, grid_for(nrec, 256), 256, 0, s, nrec, k1, hs, V, nb, seg, crow, ccol, cdiag);
     int* crp = L.crp.ensure(nV + 1, s);
     IDP_LAUNCH(k_rowptr_from_rows, grid_for(nV + 1, 256), 256, 0, s, nb, crow, nV, crp);
     L.ncb = nb;
     L.nrec = nrec;
     L.ncs = ncs;
-    IDP_HIP(hipStreamSynchronize(s));
 }
 
 void contact_gradient_gather(LinWork& L, hipStream_t s, const MeshDev& m, const double* X, const double* Xt,
@@ -2209,6 +2234,10 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     L.team_tag += (unsigned long long)A.maxit + 2;
     T.ctl = team;
     T.done = team + 3;
+    T.start = (unsigned*)(team + 3 + B);
+    // about 20 ms: other streams' kernels may hold CUs that long (IDP_TEAM_WAIT: another number of polls)
+    const char* wait = std::getenv("IDP_TEAM_WAIT");
+    T.start_limit = wait ? std::atol(wait) : 20000;
     T.nstart = handover ? nrun : 0;
     T.spin_limit = 1L << 23;
     T.aptr = L.coarse.aptr.p;
@@ -2223,9 +2252,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     hipEvent_t e0 = nullptr, e1 = nullptr;
     L.team_tok = L.prof ? L.prof->pair(e0, e1) : -1;
     if (e0) IDP_HIP(hipEventRecord(e0, s));
-    // workgroups that wait for each other have to be resident together
-    if (one) IDP_HIP(hipLaunchKernel(fn, dim3(tab.size()), dim3(TEAM_THREADS), args, 0, s));
-    else IDP_HIP(hipLaunchCooperativeKernel(fn, dim3(tab.size()), dim3(TEAM_THREADS), args, 0, s));
+    IDP_HIP(hipLaunchKernel(fn, dim3(tab.size()), dim3(TEAM_THREADS), args, 0, s));
     if (e1) IDP_HIP(hipEventRecord(e1, s));
     return true;
 }
@@ -2249,13 +2276,17 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     L.h_maxit.assign(B, 0);
     for (int i = 0; i < B; ++i)
         if (sv[i] != 2) L.h_it0[i] = 0;
-    const unsigned char* solve = L.solve_d.upload_get(sv.data(), B, s);
+    // (null: the one solve of a plain mesh, a new one)
+    const unsigned char* solve = B == 1 && sv[0] == 1 ? nullptr : L.solve_d.upload_get(sv.data(), B, s);
     const double nnzb = (double)m.nnzb_e + (double)L.ncb;
-    int* err = L.err.ensure(2 * (size_t)B + 2, s);
+    // scalars, error and state flags and the team kernel's control words,
+    // hand-over counts and start words, in one piece: they are read back together
+    const int nteam = 3 + 2 * B;
+    const size_t nints = 2 * (size_t)B + 2 + nteam, nres = 3 * (size_t)B + 3;
+    double* scal = L.scal.ensure(nres + (nints + 1) / 2, s);
+    int* err = (int*)(scal + nres);
     int* flag = err + B;
-    // team kernel: control words and per-instance hand-over counts
-    const int nteam = 3 + B;
-    int* team = L.team.ensure(nteam, s);
+    int* team = err + 2 * B + 2;
     IDP_LAUNCH(k_pcg_start, grid_for(std::max(B, nteam), 256), 256, 0, s, B, solve, flag, err, nteam, team);
     const bool haveC = L.ncb > 0;
     Profiler* P = L.prof;
@@ -2322,13 +2353,21 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     A.bpbeg = I.pcg_upd.pbeg.p;
     // launch tables over the instances that solve (re-made as instances stop)
     std::vector<int> hf(2 * B);
-    IDP_HIP(hipMemcpyAsync(hf.data(), err, 2 * B * sizeof(int), hipMemcpyDeviceToHost, s));
-    IDP_HIP(hipStreamSynchronize(s));
     std::vector<char> run(B);
-    for (int i = 0; i < B; ++i) run[i] = hf[B + i] == 0;
+    for (int i = 0; i < B; ++i) run[i] = sv[i] != 0;  // as k_pcg_start sets the flags
     int nA = 0, nB = 0;
     double frac = 1.0;  // launched share of the rows (exact for one instance, row-proportional otherwise)
     auto tables = [&]() {
+        if (B == 1 && run[0]) {  // one instance spans the launch: no table is read
+            nA = A.nbA;
+            nB = A.nbB;
+            A.nbl_upd = nB;
+            A.atab = A.btab = nullptr;
+            A.aoff = A.boff = nullptr;
+            A.ident = L.h_it0[0] + 1;  // iteration offset + 1
+            return;
+        }
+        A.ident = 0;
         auto fill = [&](const SegDev& sd, std::vector<int4>& out, std::vector<int>& off) {
             out.clear();
             off.clear();
@@ -2351,8 +2390,6 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         A.btab = L.btab.upload_get(L.h_btab.data(), L.h_btab.size(), s);
         A.aoff = L.aoff.upload_get(L.h_aoff.data(), L.h_aoff.size(), s);
         A.boff = L.boff.upload_get(L.h_boff.data(), L.h_boff.size(), s);
-        // iteration offset + 1 when one instance spans the launch (0: use the tables)
-        A.ident = (B == 1 && nA == A.nbA && nB == A.nbB) ? L.h_it0[0] + 1 : 0;
     };
     A.solve = solve;
     tables();
@@ -2362,7 +2399,7 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     A.part_rz = L.part1.ensure(2 * (size_t)A.nbB + 2, s);
     A.part_rr = L.part2.ensure(2 * (size_t)A.nbB + 2, s);
     A.flag = flag;
-    A.scal = L.scal.ensure(3 * (size_t)B + 3, s);
+    A.scal = scal;
     A.rtol2 = rtol * rtol;
     A.maxit = maxit;
     // one instance with many update blocks: reduce the partials once per
@@ -2407,14 +2444,27 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     int nstart = 0;
     for (int i = 0; i < B; ++i) nstart += run[i];
     std::vector<int> hdone(B, 0);
-    const bool teamed = nA > 0 && !A.red && shape.g == 8 && pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
+    bool teamed = nA > 0 && !A.red && shape.g == 8 && pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
     if (teamed) {
-        std::vector<int> ht(3 + B);
-        IDP_HIP(hipMemcpyAsync(hf.data(), err, 2 * B * sizeof(int), hipMemcpyDeviceToHost, s));
-        IDP_HIP(hipMemcpyAsync(ht.data(), team, ht.size() * sizeof(int), hipMemcpyDeviceToHost, s));
+        double* h = L.pin.as<double>(nres + (nints + 1) / 2);
+        IDP_HIP(hipMemcpyAsync(h, scal, (nres + (nints + 1) / 2) * sizeof(double), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
-        if (ht[0]) throw HipError(IDP_E_HIP, "PCG: a workgroup's wait for its team ran out");
-        for (int i = 0; i < B; ++i) hdone[i] = ht[3 + i];
+        const int* hi = (const int*)(h + nres);
+        if (hi[2 * B + 2]) throw HipError(IDP_E_HIP, "PCG: a workgroup's wait for its team ran out");
+        std::copy(h, h + 3 * B, hs.begin());
+        std::copy(hi, hi + 2 * B, hf.begin());
+        bool left = false;
+        for (int i = 0; i < B; ++i) {
+            hdone[i] = hi[2 * B + 2 + 3 + i];
+            run[i] = run[i] && hf[B + i] == 0 && hdone[i] == 0;  // its team did not start
+            left |= run[i] != 0;
+        }
+        if (left) {
+            teamed = false;
+            tables();
+        } else if (P) {
+            P->end(IDP_K_PCG, tok);
+        }
     }
     int it_half = -1, it_end = INT_MAX;
     int it = 0, chunk = 8;
@@ -2436,17 +2486,16 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         }
         IDP_HIP(hipMemcpyAsync(hf.data(), err, 2 * B * sizeof(int), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
-        bool all = true, fewer = false;
+        bool fewer = false;
         int nrun = 0;
         for (int i = 0; i < B; ++i) {
-            all &= hf[B + i] != 0;
             if (run[i] && hf[B + i] != 0) {
                 run[i] = 0;
                 fewer = true;
             }
             nrun += run[i];
         }
-        if (all || it > maxit) break;
+        if (nrun == 0 || it > maxit) break;
         if (handover && nstart > 1 && it_half < 0 && 2 * nrun <= nstart) {
             it_half = it;
             it_end = 2 * it;
@@ -2455,9 +2504,11 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         if (fewer) tables();  // the stream is idle here: the tables may be rewritten
         chunk = std::min(chunk * 2, 256);
     }
-    if (P) P->end(IDP_K_PCG, tok);
-    IDP_HIP(hipMemcpyAsync(hs.data(), A.scal, 3 * B * sizeof(double), hipMemcpyDeviceToHost, s));
-    IDP_HIP(hipStreamSynchronize(s));
+    if (!teamed) {
+        if (P) P->end(IDP_K_PCG, tok);
+        IDP_HIP(hipMemcpyAsync(hs.data(), A.scal, 3 * B * sizeof(double), hipMemcpyDeviceToHost, s));
+        IDP_HIP(hipStreamSynchronize(s));
+    }
     int maxdone = 0;
     double done_iters = 0;
     for (int i = 0; i < B; ++i) {
@@ -2465,8 +2516,8 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         iters[i] = 0;
         relres[i] = 0;
         if (f == 0) {
-            const int did = teamed ? hdone[i] : it;
-            if (teamed ? did == 0 : it < it_end) throw HipError(IDP_E_HIP, "PCG did not stop");
+            const int did = hdone[i] ? hdone[i] : it;
+            if (!hdone[i] && (teamed || it < it_end)) throw HipError(IDP_E_HIP, "PCG did not stop");
             iters[i] = PCG_HANDED_OVER;  // continues in the next call
             L.h_it0[i] += did;
             maxdone = std::max(maxdone, did);
@@ -2517,10 +2568,10 @@ double dev_dot(LinWork& L, hipStream_t s, long n, const double* a, const double*
     double* part = L.part3.ensure(nblk + 1, s);
     IDP_LAUNCH(k_dot_parts, nblk, RB, 0, s, n, a, b, part);
     IDP_LAUNCH(k_sum_partials, 1, RB, 0, s, nblk, part, part + nblk);
-    double v;
-    IDP_HIP(hipMemcpyAsync(&v, part + nblk, sizeof(double), hipMemcpyDeviceToHost, s));
+    double* v = L.pin.as<double>(1);
+    IDP_HIP(hipMemcpyAsync(v, part + nblk, sizeof(double), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
-    return v;
+    return *v;
 }
 
 void dev_axpy(hipStream_t s, long n, const double* a, double sc, const double* b, double* x)

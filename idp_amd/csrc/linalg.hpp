@@ -47,8 +47,7 @@ struct LinWork {
     DBuf<double> evals, cvals;
     // PCG
     DBuf<double> pinv, r, z, p, p1, q, part0, part1, part2, part3, part_bx, scal, scal2, red;
-    DBuf<int> err;
-    DBuf<int> team, team_it0;  // words of the one-kernel solve, iterations of earlier calls
+    DBuf<int> team_it0;  // one-kernel solve: iterations of earlier calls
     DBuf<int4> team_tab;
     DBuf<unsigned long long> team_words;
     unsigned long long team_tag = 0;  // last tag used in them
@@ -57,6 +56,7 @@ struct LinWork {
     DBuf<int> cl_best, cl_root, cl_size, cl_root2, cl_cnt, cl_mem, cl_cm4;
     DBuf<unsigned long long> cl_pack;
     Profiler* prof = nullptr;
+    PinBuf pin;  // results read back
     CoarseWork coarse;
     const double* xpos = nullptr;  // positions of the system being solved (coarse aggregation); null: none
 };

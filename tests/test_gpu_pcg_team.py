@@ -79,3 +79,23 @@ def test_batch_of_many_small_meshes_in_one_kernel():
         assert np.array_equal(Xa, Xm) and np.array_equal(va, vm)
         a.close()
     b.close()
+
+
+def test_a_team_that_does_not_start_leaves_the_solve_to_the_two_kernels(monkeypatch):
+    """With no patience for workgroups that are not resident yet, the first
+    workgroup leaves and the solve runs in the two-kernel loop: same bits."""
+    sc = _scene(20, 4, 4)
+
+    def solve(cv):
+        d = driver.TetAnimFix(sc)
+        r = d.ctx.newton_direction(sc.X, sc.target, sc.h, d.dHat2, d.kappa[0], coarse_verts=cv)
+        d.close()
+        return r
+
+    for cv in (-1, 48):
+        g0, s0, _, i0 = solve(cv)
+        monkeypatch.setenv("IDP_TEAM_WAIT", "0")
+        say(f"[pcg team] coarse {cv}: no wait for the team")
+        g1, s1, _, i1 = solve(cv)
+        monkeypatch.delenv("IDP_TEAM_WAIT")
+        assert i0 == i1 and np.array_equal(g0, g1) and np.array_equal(s0, s1)
