@@ -1458,6 +1458,8 @@ int idp_ctx_create(int device, idp_ctx** out)
         c->prof.s = c->s;
         c->cw.prof = &c->prof;
         c->L.prof = &c->prof;
+        c->L.pin = &c->pin;
+        c->cw.pin = &c->pin;
         // SpMV launch shape override (tuning runs): an index into the shape table
         if (const char* e = std::getenv("IDP_SPMV_SHAPE")) {
             const int k = std::atoi(e);

@@ -661,7 +661,7 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
     const int nbox = std::min(grid_for(nV, 256), 64);
     double* dbox = C.box.ensure(7 * (size_t)nbox, s);
     IDP_LAUNCH(k_coarse_box, nbox, 256, 0, s, nV, X, m.proj_mask(), dbox);
-    double* hb = L.pin.as<double>(7 * (size_t)nbox);
+    double* hb = L.pin->as<double>(7 * (size_t)nbox);
     IDP_HIP(hipMemcpyAsync(hb, dbox, 7 * (size_t)nbox * sizeof(double), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -690,8 +690,9 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
     }
     if (!(hcell > 0)) return false;
     // vertices per voxel; larger voxels while there are too many of them
-    unsigned* key = C.ckey0.ensure(nV, s);
-    unsigned* vert = C.cval0.ensure(nV, s);
+    constexpr unsigned MAX_CELLS = 65536;
+    unsigned* key = C.cells.ensure(4 * (size_t)nV + MAX_CELLS, s);
+    unsigned* vert = key + nV;
     std::vector<unsigned> cnt;
     CoarseGrid g;
     unsigned ncell = 0;
@@ -705,15 +706,15 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
             g.n[d] = (int)std::min(nd, 1e9);
         }
         g.h = hcell;
-        if (cells > 65536.0) {
-            hcell *= std::cbrt(cells / 65536.0) * 1.05;
+        if (cells > MAX_CELLS) {
+            hcell *= std::cbrt(cells / MAX_CELLS) * 1.05;
             continue;
         }
         ncell = (unsigned)cells;
-        unsigned* dc = C.ccnt.ensure(ncell, s);
+        unsigned* dc = key + 4 * (size_t)nV;
         IDP_LAUNCH(k_coarse_zero, grid_for(ncell, 256), 256, 0, s, (long)ncell, dc);
         IDP_LAUNCH(k_coarse_cells, grid_for(nV, 256), 256, 0, s, nV, X, m.proj_mask(), g, ncell, key, vert, dc);
-        unsigned* hc = L.pin.as<unsigned>(ncell);
+        unsigned* hc = L.pin->as<unsigned>(ncell);
         IDP_HIP(hipMemcpyAsync(hc, dc, ncell * sizeof(unsigned), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
         cnt.assign(hc, hc + ncell);
@@ -752,8 +753,8 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
     C.nfree = (int)nfree;
     C.aptr.upload(aptr.data(), aptr.size(), s);
     // vertices by voxel, in vertex order (Dirichlet ones last), and the modes
-    unsigned* key1 = C.ckey1.ensure(nV, s);
-    unsigned* vert1 = C.cval1.ensure(nV, s);
+    unsigned* key1 = key + 2 * (size_t)nV;
+    unsigned* vert1 = key + 3 * (size_t)nV;
     int cbits = 1;
     while (cbits < 31 && (ncell >> cbits)) ++cbits;
     sort_pairs(s, C.tmp, key, key1, vert, vert1, nV, cbits);
@@ -799,7 +800,7 @@ bool coarse_setup(LinWork& L, hipStream_t s, const MeshDev& m, const double* X)
                    D + ((k + 1) & 1) * SW * SW, info);
         std::swap(src, dst);
     }
-    int* hinfo = L.pin.as<int>(1);
+    int* hinfo = L.pin->as<int>(1);
     IDP_HIP(hipMemcpyAsync(hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
     if (*hinfo != 0) return false;  // not positive definite: no coarse level this time

@@ -348,7 +348,7 @@ __device__ inline unsigned lower_bound_u(const unsigned* a, unsigned n, unsigned
 // table per record key (all zero between calls: entries are cleared after use).
 struct CellTable {
     const unsigned* keys;
-    const int* vals;
+    const int4* recs;  // {primitive, lowest voxel of its box (clamped)}
     const unsigned* start;  // null: binary search in keys
     const unsigned* end;
     unsigned n;
@@ -363,6 +363,19 @@ __device__ inline void cell_range(const CellTable& T, unsigned key, unsigned& s,
         s = lower_bound_u(T.keys, T.n, key);
         e = lower_bound_u(T.keys, T.n, key + 1);
     }
+}
+
+// the sorted records with the box minimum that the walks test beside each
+// primitive: one 16-byte load per record instead of the primitive and then
+// its box
+__global__ void k_cell_recs(unsigned n, const unsigned* __restrict__ keys, const int* __restrict__ vals, int nsplit,
+                            const int* __restrict__ pbox, int4* __restrict__ recs)
+{
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int f = vals[i];
+    const int* pb = pbox + 6L * (f + ((keys[i] & 1u) ? nsplit : 0));  // key bases are even: the type is the low bit
+    recs[i] = make_int4(f, max(pb[0], 0), max(pb[1], 0), max(pb[2], 0));
 }
 
 // sets (clear = 0) or resets (clear = 1) the table entries of the keys present
@@ -412,14 +425,12 @@ struct WalkLane {
         li = (unsigned)lane;
     }
     // the next primitive found by this lane; -1 at the end
-    __device__ int next(const CellTable& T, const int* __restrict__ pbox_t)
+    __device__ int next(const CellTable& T)
     {
         for (;;) {
             while (k < e) {
-                const int f = T.vals[k++];
-                const int* pb = pbox_t + 6L * f;
-                if (max(q[0], max(pb[0], 0)) == x && max(q[1], max(pb[1], 0)) == y && max(q[2], max(pb[2], 0)) == z)
-                    return f;
+                const int4 c = T.recs[k++];
+                if (max(q[0], c.y) == x && max(q[1], c.z) == y && max(q[2], c.w) == z) return c.x;
             }
             if (li >= nvox) return -1;
             x = l[0] + (int)(li % (unsigned)n[0]);
@@ -671,7 +682,6 @@ __global__ void __launch_bounds__(256) k_cs_walk(int nb, int ne, CSArgs A, CellT
     WalkLane<G> W;
     W.none();
     int eI = -1;  // edge queries take edges of larger index only
-    const int* pbox = A.pbox;
     if (q < (long)nb + ne) {
         int ql[3], qh[3], inst, type = 0;
         double r;
@@ -693,7 +703,6 @@ __global__ void __launch_bounds__(256) k_cs_walk(int nb, int ne, CSArgs A, CellT
             locate(g, fmin(a.x, b.x) - r, fmin(a.y, b.y) - r, fmin(a.z, b.z) - r, ql);
             locate(g, fmax(a.x, b.x) + r, fmax(a.y, b.y) + r, fmax(a.z, b.z) + r, qh);
             type = 1;
-            pbox = A.pbox + 6L * A.nf;
         }
         if (!(A.active && !A.active[inst])) W.start(A.grids[inst], A.keybase[inst], type, ql, qh, lane);
     }
@@ -709,7 +718,7 @@ __global__ void __launch_bounds__(256) k_cs_walk(int nb, int ne, CSArgs A, CellT
         }
     };
     for (;;) {
-        const int f = W.next(T, pbox);
+        const int f = W.next(T);
         if (__ballot(f >= 0) == 0) break;
         Q.push(f > eI, make_int2((int)q, f), test);
     }
@@ -847,14 +856,10 @@ __global__ void __launch_bounds__(256) k_ccd_walk(int nb, int ne, CCDArgs A, Cel
         WalkLane<G> W;
         W.none();
         int eI = -1;  // edge queries take edges of larger index only
-        const int* pbox = A.pbox;
         if (q >= 0) {
             const int* box = q < nb ? A.vbox + 6 * q : pe + 6 * (q - nb);
             const int inst = A.vinst[q < nb ? A.bn[q] : A.be[q - nb].x];
-            if (q >= nb) {
-                eI = (int)(q - nb);
-                pbox = pe;
-            }
+            if (q >= nb) eI = (int)(q - nb);
             if (!(A.active && !A.active[inst])) {
                 const GridDev& g = A.grids[inst];
                 if (!BIG && walk_nvox(g, box, box + 3) > WALK_BIG_VOX) {
@@ -865,7 +870,7 @@ __global__ void __launch_bounds__(256) k_ccd_walk(int nb, int ne, CCDArgs A, Cel
             }
         }
         for (;;) {
-            const int f = W.next(T, pbox);
+            const int f = W.next(T);
             if (__ballot(f >= 0) == 0) break;
             Q.push(f > eI, make_int2((int)q, f), test);
         }
@@ -1362,7 +1367,7 @@ CellTable build_cells(ContactWork& w, hipStream_t s, const MeshDev& m, const int
                w.grids.p, pbox + 6 * (size_t)m.nf, cnt + m.nf, pinst + m.nf);
     IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, cnt + n, 1);
     excl_scan(s, w.tmp, cnt, off, n + 1);
-    GridDev* hg = w.pin.as<GridDev>(B + 1);
+    GridDev* hg = w.pin->as<GridDev>(B + 1);
     unsigned* htotal = (unsigned*)(hg + B);
     IDP_HIP(hipMemcpyAsync(htotal, off + n, sizeof(unsigned), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipMemcpyAsync(hg, w.grids.p, B * sizeof(GridDev), hipMemcpyDeviceToHost, s));
@@ -1394,7 +1399,9 @@ CellTable build_cells(ContactWork& w, hipStream_t s, const MeshDev& m, const int
     const unsigned long long nkeys = acc;
     sort_pairs(s, w.tmp, k0, k1, v0, v1, total, bits_for(nkeys));
     T.keys = k1;
-    T.vals = v1;
+    int4* recs = w.recs.ensure(total, s);
+    IDP_LAUNCH(k_cell_recs, grid_for(total, 256), 256, 0, s, total, k1, v1, m.nf, pbox, recs);
+    T.recs = recs;
     if (nkeys <= DENSE_MAX) {
         if (w.cstart.cap < nkeys || !w.cstart.p) {
             w.cstart.ensure(nkeys, s);
@@ -1509,7 +1516,7 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
             if (G == 32) IDP_LAUNCH(k_cs_walk<32>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
             else if (G == 16) IDP_LAUNCH(k_cs_walk<16>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
             else IDP_LAUNCH(k_cs_walk<8>, wb, 256, 0, s, m.nb, m.ne, A, T, O);
-            unsigned* h = w.pin.as<unsigned>(2);
+            unsigned* h = w.pin->as<unsigned>(2);
             IDP_HIP(hipMemcpyAsync(h, cnt, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, s));
             IDP_HIP(hipStreamSynchronize(s));
             hc[0] = h[0];
@@ -1541,7 +1548,7 @@ long contact_constraint_set(ContactWork& w, hipStream_t s, const MeshDev& m, con
         IDP_LAUNCH(k_dup_heads, grid_for(nd, 256), 256, 0, s, nd, k1, head);
         IDP_LAUNCH(k_zero_u32, 1, 64, 0, s, head + nd, 1);
         excl_scan(s, w.tmp, head, hs, nd + 1);
-        nmerged = read_u(w.pin, s, hs + nd);
+        nmerged = read_u(*w.pin, s, hs + nd);
         int4* mout = direct ? w.cs.p + npass : w.merged.ensure(nmerged + 1, s);
         IDP_LAUNCH(k_dup_write, grid_for(nd, 256), 256, 0, s, nd, k1, hs, I.d_vbeg.p, O.inst_shift, mout);
     }
@@ -1716,7 +1723,7 @@ void contact_ccd_batch(ContactWork& w, hipStream_t s, const MeshDev& m, const do
             IDP_HIP(hipEventDestroy(e0));
             IDP_HIP(hipEventDestroy(e1));
         }
-        unsigned long long* h = w.pin.as<unsigned long long>((size_t)B + 7);
+        unsigned long long* h = w.pin->as<unsigned long long>((size_t)B + 7);
         IDP_HIP(hipMemcpyAsync(h, amin, ((size_t)B + 7) * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
         std::copy(h, h + B, ha.begin());

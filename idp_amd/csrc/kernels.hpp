@@ -135,6 +135,7 @@ struct ContactWork {
     DBuf<unsigned> u0, u1, cP, cD, oP, oD, k0, k1;
     DBuf<int> v0, v1;
     DBuf<int4> pass, dup, merged, cs;
+    DBuf<int4> recs;  // sorted cell records
     DBuf<unsigned long long> dk0, dk1, pk0, pk1;
     DBuf<unsigned> cstart, cend, cnt;  // dense cell table, atomic counters
     DBuf<int2> cand;
@@ -165,7 +166,7 @@ struct ContactWork {
     bool accd_cert = true;    // long ACCD pairs try the no-hit certificate
     std::vector<unsigned> h_capped;  // ... per instance
     DBuf<unsigned> icap;
-    PinBuf pin;                        // results read back
+    PinBuf* pin = nullptr;             // results read back (the context's)
     std::vector<double> h_rad;         // what rad and keybase hold
     std::vector<unsigned> h_keybase;
     Profiler* prof = nullptr;

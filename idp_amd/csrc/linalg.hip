@@ -2061,7 +2061,7 @@ void contact_structure(LinWork& L, hipStream_t s, int nV, long ncs0, const int* 
     IDP_LAUNCH(k_contact_nv2, grid_for(ncs, 256), 256, 0, s, ncs, nv, cnt);
     IDP_HIP(hipMemsetAsync(cnt + ncs, 0, sizeof(unsigned), s));
     excl_scan<unsigned>(s, L.tmp, cnt, off, (int)ncs + 1);
-    unsigned nrec = read_u(L.pin, s, off + ncs);
+    unsigned nrec = read_u(*L.pin, s, off + ncs);
     unsigned long long V = (unsigned long long)nV;
     unsigned long long* k0 = L.key0.ensure(nrec, s);
     unsigned* v0 = L.rv0.ensure(nrec, s);
@@ -2073,7 +2073,7 @@ void contact_structure(LinWork& L, hipStream_t s, int nV, long ncs0, const int* 
     unsigned* hs = L.u1.ensure(nrec + 1, s);
     IDP_LAUNCH(k_run_heads, grid_for(nrec + 1, 256), 256, 0, s, nrec, k1, head);
     excl_scan<unsigned>(s, L.tmp, head, hs, (int)nrec + 1);
-    unsigned nb = read_u(L.pin, s, hs + nrec);
+    unsigned nb = read_u(*L.pin, s, hs + nrec);
     unsigned* seg = L.seg.ensure(nb + 1, s);
     int* crow = L.crow.ensure(nb + 1, s);
     int* ccol = L.ccol.ensure(nb + 1, s);
@@ -2444,9 +2444,10 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     int nstart = 0;
     for (int i = 0; i < B; ++i) nstart += run[i];
     std::vector<int> hdone(B, 0);
-    bool teamed = nA > 0 && !A.red && shape.g == 8 && pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
+    // (full profiling times the two kernels by themselves, with the same results)
+    bool teamed = nA > 0 && !(P && P->full()) && !A.red && shape.g == 8 && pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
     if (teamed) {
-        double* h = L.pin.as<double>(nres + (nints + 1) / 2);
+        double* h = L.pin->as<double>(nres + (nints + 1) / 2);
         IDP_HIP(hipMemcpyAsync(h, scal, (nres + (nints + 1) / 2) * sizeof(double), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
         const int* hi = (const int*)(h + nres);
@@ -2568,7 +2569,7 @@ double dev_dot(LinWork& L, hipStream_t s, long n, const double* a, const double*
     double* part = L.part3.ensure(nblk + 1, s);
     IDP_LAUNCH(k_dot_parts, nblk, RB, 0, s, n, a, b, part);
     IDP_LAUNCH(k_sum_partials, 1, RB, 0, s, nblk, part, part + nblk);
-    double* v = L.pin.as<double>(1);
+    double* v = L.pin->as<double>(1);
     IDP_HIP(hipMemcpyAsync(v, part + nblk, sizeof(double), hipMemcpyDeviceToHost, s));
     IDP_HIP(hipStreamSynchronize(s));
     return *v;

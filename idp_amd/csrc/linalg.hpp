@@ -17,7 +17,7 @@ struct CoarseWork {
     int K = 0, ncd = 0, lda = 0, nsb = 0, nfree = 0;  // lda: leading dimension of A_c^-1
     DBuf<int> agg, aptr, avert;
     DBuf<double> P, Ainv, Awork, diag, box, rc, part;
-    DBuf<unsigned> ckey0, ckey1, cval0, cval1, ccnt;  // voxels of the vertices
+    DBuf<unsigned> cells;  // voxel and id of every vertex, twice (sort), then the vertices per voxel
     DBuf<double> Ps;  // P in aggregate order: 18 planes over the slots of avert
     DBuf<unsigned long long> key0, key1;
     DBuf<unsigned> val0, val1, head, hs, seg;
@@ -56,7 +56,7 @@ struct LinWork {
     DBuf<int> cl_best, cl_root, cl_size, cl_root2, cl_cnt, cl_mem, cl_cm4;
     DBuf<unsigned long long> cl_pack;
     Profiler* prof = nullptr;
-    PinBuf pin;  // results read back
+    PinBuf* pin = nullptr;  // results read back (the context's)
     CoarseWork coarse;
     const double* xpos = nullptr;  // positions of the system being solved (coarse aggregation); null: none
 };
