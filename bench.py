@@ -609,7 +609,14 @@ def bench_plain(a):
     d.ctx.profile(0)
     roof = _roofline("pcg_spmv", prof_t, a.traffic)
     extra = {"roofline": roof}
-    extra["roofline_update_kernel"] = _roofline("pcg_update", prof_t, a.traffic)
+    # a system of up to 32,768 rows is solved by one kernel per solve: its time
+    # and the bytes of all its iterations are the SpMV family's record, and there
+    # is no update kernel
+    if prof_t["pcg_update"]["launches"]:
+        extra["roofline_update_kernel"] = _roofline("pcg_update", prof_t, a.traffic)
+    elif roof:
+        roof["kernel"] = "pcg_team"
+        roof["traffic"] = None
     state["extra"] = extra
 
     # per-family device times: a profiled solve truncated to a bounded number
