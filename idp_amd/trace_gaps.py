@@ -22,7 +22,7 @@ import sys
 
 import numpy as np
 
-PCG_KERNELS = ("k_pcg_spmv", "k_pcg_update", "k_pcg_red_spmv", "k_pcg_red_upd", "k_coarse_restrict", "k_coarse_solve")
+PCG_KERNELS = ("k_pcg_team", "k_pcg_spmv", "k_pcg_update", "k_pcg_red_spmv", "k_pcg_red_upd", "k_coarse_restrict", "k_coarse_solve")
 
 
 def _base(name):
