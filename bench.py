@@ -647,10 +647,15 @@ def bench_plain(a):
     # what a graph of the PCG iterations could remove at most: the PCG stage's
     # device time between its kernels (launch gaps, chunk-boundary waits and
     # the preconditioner build), from the sampled per-launch kernel times
+    # (one record of the SpMV family per solve, and none of the update, where
+    # a solve runs as one kernel)
     sp, up = prof["pcg_spmv"], prof["pcg_update"]
-    if sp["launches"] and up["launches"] and prof["pcg"]["ms"] > 0:
-        per_it = sp["ms"] / sp["launches"] + up["ms"] / up["launches"]
-        kms = per_it * st_p["pcg_iters"]
+    if sp["launches"] and prof["pcg"]["ms"] > 0:
+        if up["launches"]:
+            kms = (sp["ms"] / sp["launches"] + up["ms"] / up["launches"]) * st_p["pcg_iters"]
+        else:
+            kms = sp["ms"]
+            kern["pcg"]["solve_kernels"] = "one per solve"
         kern["pcg"]["iterations"] = int(st_p["pcg_iters"])
         kern["pcg"]["kernel_ms_est"] = kms
         kern["pcg"]["outside_kernels_ms"] = prof["pcg"]["ms"] - kms

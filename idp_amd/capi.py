@@ -676,6 +676,7 @@ class Context:
         return X.reshape(-1, 3), v.reshape(-1, 3)
 
     def profile(self, on=True):
+        """Level 0 to 3 (see idp_profile_enable); 3 runs the PCG in its two-kernel loop."""
         self._check(lib().idp_profile_enable(self._h, int(on)))
 
     def profile_read(self):

@@ -1534,7 +1534,7 @@ int idp_get_launch_config(idp_ctx* c, int* spmv_shape, int* upd_waves)
 int idp_profile_enable(idp_ctx* c, int on)
 {
     return guarded(c, [&]() -> int {
-        if (on < 0 || on > 2) return IDP_E_INVALID;
+        if (on < 0 || on > 3) return IDP_E_INVALID;
         c->prof.reset();
         c->prof.level = on;
         c->prof.on = on != 0;

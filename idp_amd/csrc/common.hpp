@@ -177,10 +177,12 @@ struct Profiler {
         double work;
     };
     // 0 off; 1 every family (an event pair around each launch); 2 only the
-    // sampled PCG kernel pairs, so a timed run keeps its launch gaps
+    // sampled PCG kernel pairs, so a timed run keeps its launch gaps; 3 as 1,
+    // with every PCG solve in the two-kernel loop
     int level = 0;
     bool on = false;  // level != 0
-    bool full() const { return level == 1; }
+    bool full() const { return level == 1 || level == 3; }
+    bool two_kernels() const { return level == 3; }
     hipStream_t s = nullptr;
     std::vector<hipEvent_t> pool;
     std::vector<Rec> open;

@@ -2444,8 +2444,8 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     int nstart = 0;
     for (int i = 0; i < B; ++i) nstart += run[i];
     std::vector<int> hdone(B, 0);
-    // (full profiling times the two kernels by themselves, with the same results)
-    bool teamed = nA > 0 && !(P && P->full()) && !A.red && shape.g == 8 && pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
+    bool teamed = nA > 0 && !(P && P->two_kernels()) && !A.red && shape.g == 8 &&
+                  pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
     if (teamed) {
         double* h = L.pin->as<double>(nres + (nints + 1) / 2);
         IDP_HIP(hipMemcpyAsync(h, scal, (nres + (nints + 1) / 2) * sizeof(double), hipMemcpyDeviceToHost, s));

@@ -112,8 +112,8 @@ enum {
     IDP_K_CCD = 5,          /* ACCD kernel over candidate pairs (pair count) */
     IDP_K_ENERGY = 6,       /* tet + inertia + barrier energy kernels */
     IDP_K_GRADIENT = 7,     /* tet + barrier gradient and vertex gather */
-    IDP_K_PCG_SPMV = 8,     /* PCG SpMV kernel, sampled on one iteration in 8, or (level 2) the whole solve
-                               where it runs as one kernel (bytes) */
+    IDP_K_PCG_SPMV = 8,     /* PCG SpMV kernel, sampled on one iteration in 8, or the whole solve where
+                               it runs as one kernel (bytes) */
     IDP_K_PCG_UPDATE = 9,   /* PCG vector-update kernel, sampled likewise (bytes) */
     IDP_K_FRICTION = 10,    /* friction Hessian kernel (bytes) */
     IDP_K_FRICTION_BASIS = 11, /* friction basis update: flags, scan, records (bytes) */
@@ -145,8 +145,10 @@ int idp_device_memory(long long* in_use, long long* peak);
  * family (an event pair around each launch, constraint-kind counters in the
  * barrier Hessian); on = 2 records only the PCG SpMV and update kernels on
  * one iteration in eight, which leaves the launch stream as it runs
- * unprofiled (a solve that runs as one kernel is one SpMV record; level 1
- * runs every solve in the two kernels); on = 0 stops. */
+ * unprofiled; on = 3 records as on = 1 and runs every PCG solve in the two
+ * kernels, with the same results, so that both are timed on any mesh; on = 0
+ * stops.  Where a solve runs as one kernel (up to 32,768 rows, on = 1 or 2)
+ * it is one SpMV record and no update record. */
 int idp_profile_enable(idp_ctx* ctx, int on);
 int idp_profile_read(idp_ctx* ctx, idp_profile* out);
 /* Launch configuration of the PCG kernels (no counterpart in the reference;

@@ -99,3 +99,33 @@ def test_a_team_that_does_not_start_leaves_the_solve_to_the_two_kernels(monkeypa
         g1, s1, _, i1 = solve(cv)
         monkeypatch.delenv("IDP_TEAM_WAIT")
         assert i0 == i1 and np.array_equal(g0, g1) and np.array_equal(s0, s1)
+
+
+def _direction(d, sc, level, coarse=-1, X=None):
+    """One Newton direction at a profile level; (gradient, direction, PCG
+    iterations, one-kernel solves, launches of the update kernel seen)."""
+    d.ctx.profile(level)
+    g, s, r, it = d.ctx.newton_direction(sc.X if X is None else X, sc.target, sc.h, d.dHat2, d.kappa[0],
+                                         pcg_rtol=1e-10, coarse_verts=coarse)
+    p = d.ctx.profile_read()
+    d.ctx.profile(0)
+    assert r <= 1e-10
+    return g, s, it, p["pcg_spmv"]["launches"], p["pcg_update"]["launches"]
+
+
+def test_profiles_record_the_solve_that_runs():
+    """Levels 1 and 2 record the one-kernel solve of a program that does not
+    profile; level 3 runs the two kernels, which are then seen, with the same
+    result."""
+    sc = _scene(12, 4, 2)
+    d = driver.TetAnimFix(sc)
+    try:
+        runs = {level: _direction(d, sc, level) for level in (1, 2, 3)}
+        for level in (1, 2):
+            assert runs[level][3:] == (1, 0), (level, runs[level][3:])
+        assert runs[3][3] >= 1 and runs[3][4] >= 1
+        for level in (2, 3):
+            assert runs[level][2] == runs[1][2]
+            assert np.array_equal(runs[level][0], runs[1][0]) and np.array_equal(runs[level][1], runs[1][1])
+    finally:
+        d.close()
