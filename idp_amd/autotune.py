@@ -1,7 +1,9 @@
 """Autotuner for the launch configuration on this device.
 
-The PCG runs two kernels per iteration.  Two of its launch parameters are
-tuned:
+Above 32,768 rows the PCG runs two kernels per iteration (smaller systems run
+as one kernel per solve, which has no parameters).  Two launch parameters of
+the two kernels are tuned, on any workload with the PCG held to them (profile
+level 3):
 - the SpMV shape (index into the library's table: G = 4, 8, 16, 32 lanes per
   block row, with the scalar reduction in wavefront 0 for 0..3 or in a fifth
   wavefront for 4..7);
@@ -9,7 +11,11 @@ tuned:
 
 The two kernels are timed separately (kernel-accurate HIP events on sampled
 iterations), so the search is separable: every SpMV shape at the default
-update width, then every update width at the best shape.  The objective is
+update width, then every update width at the best shape of 8 lanes per row.
+The one-kernel solve adds each row as 8 lanes do, so another G would take it
+away from every smaller mesh (24 us per iteration instead of 5 on 81 rows, far
+more than the shapes differ); the other shapes are measured and recorded, and
+a faster one is named in the log.  The objective is
 the kernel time per PCG iteration, summed over the workloads given, because
 the iteration count itself moves slightly with G (G sets the order of each
 block row's sum).  For the same reason the result is one configuration for
@@ -39,6 +45,7 @@ from . import capi, driver, scenes
 SHAPE_TABLE = [(4, False), (8, False), (16, False), (32, False), (4, True), (8, True), (16, True), (32, True)]
 UPD_WAVES = [1, 2, 4, 8]
 DEFAULT = (5, 4)
+TEAM_LANES = 8  # lanes per row whose sums the one-kernel PCG solve forms
 TEAMS = [3, 8, 16, 32, 64]
 DEFAULT_TEAM = 3
 
@@ -59,7 +66,7 @@ def measure(kind, sc, spmv_shape, upd_waves, newton):
     first `newton` Newton iterations of one step."""
     d = driver.TetAnimFix(sc) if kind == "one" else driver.BatchAnimFix(sc)
     d.ctx.set_launch_config(spmv_shape, upd_waves)
-    d.ctx.profile(True)
+    d.ctx.profile(3)
     its, _ = d.advance_one_time_step(max_newton=newton)
     p = d.ctx.profile_read()
     d.ctx.profile(False)
@@ -133,6 +140,11 @@ def choose(rows):
     return best_shape, best_w
 
 
+def _eligible(rows):
+    """The measurements of shapes whose row sums are those of the one-kernel solve."""
+    return [r for r in rows if SHAPE_TABLE[r["spmv_shape"]][0] == TEAM_LANES]
+
+
 def tune(workloads, newton, log=print):
     rows = []
     for name in workloads:
@@ -142,7 +154,11 @@ def tune(workloads, newton, log=print):
             r["workload"] = name
             rows.append(r)
             log(f"[tune] {name} shape {shape} {SHAPE_TABLE[shape]}: spmv {r['spmv_us']:.2f} us")
-    best_shape, _ = choose(rows)
+    best_shape, _ = choose(_eligible(rows))
+    fastest, _ = choose(rows)
+    if fastest != best_shape:
+        log(f"[tune] shape {fastest} {SHAPE_TABLE[fastest]} has the faster SpMV, but {TEAM_LANES} lanes per row keep "
+            f"the one-kernel solve of smaller meshes: shape {best_shape}")
     for name in workloads:
         kind, sc = _workload(name)
         for w in UPD_WAVES:
@@ -152,7 +168,7 @@ def tune(workloads, newton, log=print):
             r["workload"] = name
             rows.append(r)
             log(f"[tune] {name} update width {w}: update {r['update_us']:.2f} us")
-    return choose(rows), rows
+    return choose(_eligible(rows)), rows
 
 
 def main(argv=None):

@@ -65,6 +65,38 @@ def test_tune_measures_shapes_then_widths(monkeypatch):
     assert len(rows) == len(calls) and {r["workload"] for r in rows} == {"a", "b"}
 
 
+def test_tune_keeps_the_lanes_of_the_one_kernel_solve(monkeypatch):
+    """A faster SpMV shape of another lanes-per-row count is reported, not
+    chosen: it would switch the one-kernel solve off."""
+    levels, lines = [], []
+
+    class Ctx:
+        def set_launch_config(self, shape, waves):
+            self.cfg = shape, waves
+
+        def profile(self, level):
+            levels.append(level)
+
+        def profile_read(self):
+            us = {2: 5.0, 5: 9.0}.get(self.cfg[0], 20.0)
+            return {"pcg_spmv": {"ms": us * 1e-3, "launches": 1}, "pcg_update": {"ms": 1e-3, "launches": 1}}
+
+    class Driver:
+        def __init__(self, sc):
+            self.ctx = Ctx()
+
+        def advance_one_time_step(self, max_newton):
+            return 1, {}
+
+    monkeypatch.setattr(autotune.driver, "TetAnimFix", Driver)
+    monkeypatch.setattr(autotune, "_workload", lambda name: ("one", None))
+    (shape, _), rows = autotune.tune(["a"], newton=1, log=lambda *a: lines.append(" ".join(map(str, a))))
+    assert shape == 5 and autotune.SHAPE_TABLE[shape][0] == autotune.TEAM_LANES
+    assert {r["spmv_shape"] for r in rows} == set(range(len(autotune.SHAPE_TABLE)))  # the others stay on record
+    assert any("shape 2 (16, False) has the faster SpMV" in x for x in lines)
+    assert set(levels) <= {0, 3}  # the two kernels are what is timed
+
+
 def test_choose_team_sums_workloads_and_prefers_the_default():
     rows = [{"workload": "a", "barrier_team": 8, "barrier_hess_us": 30.0},
             {"workload": "a", "barrier_team": 16, "barrier_hess_us": 20.0},

@@ -1,7 +1,8 @@
 """PCG launch configuration on MI355X, through the C ABI.
 
 The update width and the placement of the scalar wavefront do not change
-any arithmetic, so results are compared bit for bit across them.  Another
+any arithmetic, so results are compared bit for bit across them (with the
+solves held to the two kernels that take them, profile level 3).  Another
 lanes-per-row count G changes the order of each block row's sum, so its
 result is compared with the oracle at the usual 1e-6 of the bounding-box
 diagonal instead.
@@ -25,7 +26,10 @@ def _solve(sc, shape, waves):
     d = driver.TetAnimFix(sc)
     d.ctx.set_launch_config(shape, waves)
     assert d.ctx.launch_config() == (shape, waves)
+    d.ctx.profile(3)
     it, st = d.advance_one_time_step()
+    p = d.ctx.profile_read()
+    assert p["pcg_spmv"]["launches"] > it and p["pcg_update"]["launches"] > it  # the two kernels ran
     X, v = d.state()
     return it, st["pcg_iters"], X, v
 
