@@ -15,7 +15,7 @@
 #include "prim.hpp"
 #include "kernels.hpp"
 #include "linalg.hpp"
-
+#include "team_rule.hpp"
 
 namespace idp {
 
@@ -1244,9 +1244,9 @@ struct TeamArgs {
     // published partials, two words each: p.q (nbA), r.z, r.r and the hand-over mark (2 nbB + B), r_c, r_c . e_c
     unsigned long long *w_pq, *w_r, *w_rc, *w_cp;
     unsigned tag0;    // tags of this launch are tag0 + 1 + iteration; larger than any before
-    int* ctl;         // [0] a wait ran out (the launch is void), [1] solves stopped, [2] hand-over after this many
-                      // iterations (0: not yet)
+    int* ctl;         // [0] a wait ran out (the launch is void)
     int* done;        // per instance: iterations done by this call when handed over
+    int* hand;        // hand-over counts (team_hand): solves past each look, solves stopped before it, solves started
     unsigned* start;  // per instance: workgroups of its team that are resident, TEAM_LEFT when one has left
     long start_limit; // polls of the wait for all of them
     int nstart;       // hand-over: solves at launch (0: never)
@@ -1357,6 +1357,27 @@ __device__ inline bool team_start(unsigned* word, unsigned size, long limit)
             return false;  // (on failure w is the word as it stands)
         if (k < limit) w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// Whether the solves still running are handed over at look k: as in the
+// two-kernel loop, when half of the launch's solves had stopped by then.  That
+// loop's solves go in step; here a solve that needs the answer, which is after
+// twice as many iterations, may have to wait until every other one is past the
+// look or has stopped.  Only solves of which all have started wait: their
+// workgroups are resident, the one furthest behind always runs, so the wait
+// ends (and is bounded like every other).  The answer does not depend on how
+// fast each runs; only where some have not started yet (other work on the GPU)
+// is it no, and the solves go on.
+__device__ inline bool team_hand(const TeamArgs& T, int k)
+{
+    if (k >= HAND_LOOKS || team_ld<false>(T.hand + 2 * HAND_LOOKS) != T.nstart) return false;
+    for (long n = 0; n < T.spin_limit / HAND_LOOKS; ++n) {
+        const int past = team_ld<false>(T.hand + k);
+        int stopped = 0;
+        for (int j = 0; j <= k; ++j) stopped += team_ld<false>(T.hand + HAND_LOOKS + j);
+        if (past + stopped == T.nstart) return 2 * past <= T.nstart;
+    }
+    return false;
 }
 
 // cross-lane moves of a double within a row of 16 lanes (DPP; an LDS
@@ -1667,6 +1688,10 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
     double* sci = A.scal + 3 * inst;
     double rz = 0.0, rr = 0.0, rzo = 1.0, bb = 0.0;
     int hand = 0;
+    // the next look of this solve (k-th) and the next look whose answer it needs
+    int look = HAND_FIRST, klook = 0, ans = HAND_FIRST, kans = 0;
+    const bool counts = T.nstart && rank == 0 && tid == 0;
+    if (counts) atomicAdd(T.hand + 2 * HAND_LOOKS, 1);
     if (tid == 0) bad = 0;
     // ---- the workgroup's blocks and update state stay in registers
     const int gl = lane & 7;
@@ -1752,16 +1777,21 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
         const unsigned tag = T.tag0 + 1u + (unsigned)(it - it_first);
         const int par = it & 1;
         // the same decisions in every workgroup of the team
+        if (hand) {
+            state = -1;
+            break;
+        }
+        if (it - it_first == look) {
+            if (counts && klook < HAND_LOOKS) atomicAdd(T.hand + klook, 1);
+            look = hand_next(look);
+            ++klook;
+        }
         if (!(bb > 0.0) || (it > 0 && rr <= A.rtol2 * bb)) {
             state = 1;
             break;
         }
         if (it >= A.maxit) {
             state = 4;
-            break;
-        }
-        if (hand) {
-            state = -1;
             break;
         }
         const double beta = it > 0 ? rz / rzo : 0.0;
@@ -1857,10 +1887,11 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
         // an odd number of blocks: the last line's other half is published too, so that all of it is waited for
         if (wave == 1 && lane < 2 && (nb & 1) && rank == size - 1)
             team_put<ONE>(w_r, nr, val, team_rblk(nb) + 2 * lane, 0.0, tag);
-        if (T.nstart && rank == 0 && tid == 0) {
-            // half of the solves have stopped: hand over after as many iterations again
-            const int half = team_ld<false>(T.ctl + 2);
-            team_put<ONE>(w_r, nr, val, nr - 1, half > 0 && it + 1 - it_first >= 2 * half ? 1.0 : 0.0, tag);
+        const bool asks = it + 1 - it_first == 2 * ans;
+        if (counts) team_put<ONE>(w_r, nr, val, nr - 1, asks && team_hand(T, kans) ? 1.0 : 0.0, tag);
+        if (asks) {
+            ans = hand_next(ans);
+            ++kans;
         }
         if (!team_meet<ONE>(T, w_r, T.nstart ? nr : nr - 1, tag, val, &bad)) return;
         if (wave == 0) {
@@ -1982,10 +2013,7 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
     A.flag[inst] = state;
     if (state != 2) sci[1] = rr;
     sci[2] = (double)it;
-    if (T.nstart) {  // once half of the solves have stopped, the others learn after how many iterations
-        const int n = atomicAdd(T.ctl + 1, 1) + 1;
-        if (2 * n >= T.nstart) atomicCAS(T.ctl + 2, 0, max(1, it - it_first));
-    }
+    if (counts && klook < HAND_LOOKS) atomicAdd(T.hand + HAND_LOOKS + klook, 1);  // stopped before its next look
 }
 
 // generic deterministic sum of partials -> out[0]
@@ -2233,8 +2261,9 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     T.tag0 = (unsigned)L.team_tag;
     L.team_tag += (unsigned long long)A.maxit + 2;
     T.ctl = team;
-    T.done = team + 3;
-    T.start = (unsigned*)(team + 3 + B);
+    T.done = team + 1;
+    T.start = (unsigned*)(team + 1 + B);
+    T.hand = team + 1 + 2 * B;
     // about 20 ms: other streams' kernels may hold CUs that long (IDP_TEAM_WAIT: another number of polls)
     const char* wait = std::getenv("IDP_TEAM_WAIT");
     T.start_limit = wait ? std::atol(wait) : 20000;
@@ -2279,9 +2308,10 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     // (null: the one solve of a plain mesh, a new one)
     const unsigned char* solve = B == 1 && sv[0] == 1 ? nullptr : L.solve_d.upload_get(sv.data(), B, s);
     const double nnzb = (double)m.nnzb_e + (double)L.ncb;
-    // scalars, error and state flags and the team kernel's control words,
-    // hand-over counts and start words, in one piece: they are read back together
-    const int nteam = 3 + 2 * B;
+    // scalars, error and state flags and the team kernel's words (void mark,
+    // iterations at a hand-over, start words, hand-over counts), in one piece:
+    // they are read back together
+    const int nteam = 1 + 2 * B + 2 * HAND_LOOKS + 1;
     const size_t nints = 2 * (size_t)B + 2 + nteam, nres = 3 * (size_t)B + 3;
     double* scal = L.scal.ensure(nres + (nints + 1) / 2, s);
     int* err = (int*)(scal + nres);
@@ -2443,7 +2473,7 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     // their state for the next call.  One solve alone is never handed over.
     int nstart = 0;
     for (int i = 0; i < B; ++i) nstart += run[i];
-    std::vector<int> hdone(B, 0);
+    std::vector<int> hdone(B, 0), tstop(B, -1);  // one-kernel solves: handed over / stopped after these iterations
     bool teamed = nA > 0 && !(P && P->two_kernels()) && !A.red && shape.g == 8 &&
                   pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
     if (teamed) {
@@ -2456,7 +2486,8 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         std::copy(hi, hi + 2 * B, hf.begin());
         bool left = false;
         for (int i = 0; i < B; ++i) {
-            hdone[i] = hi[2 * B + 2 + 3 + i];
+            hdone[i] = hi[2 * B + 2 + 1 + i];
+            if (run[i] && hf[B + i] != 0) tstop[i] = (int)hs[3 * i + 2] - L.h_it0[i];
             run[i] = run[i] && hf[B + i] == 0 && hdone[i] == 0;  // its team did not start
             left |= run[i] != 0;
         }
@@ -2488,16 +2519,17 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
         IDP_HIP(hipMemcpyAsync(hf.data(), err, 2 * B * sizeof(int), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
         bool fewer = false;
-        int nrun = 0;
+        int nrun = 0, later = 0;
         for (int i = 0; i < B; ++i) {
             if (run[i] && hf[B + i] != 0) {
                 run[i] = 0;
                 fewer = true;
             }
             nrun += run[i];
+            later += tstop[i] >= it;  // stopped, in the one kernel, after more iterations
         }
         if (nrun == 0 || it > maxit) break;
-        if (handover && nstart > 1 && it_half < 0 && 2 * nrun <= nstart) {
+        if (handover && nstart > 1 && it_half < 0 && 2 * (nrun + later) <= nstart) {
             it_half = it;
             it_end = 2 * it;
         }

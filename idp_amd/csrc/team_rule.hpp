@@ -1,0 +1,21 @@
+// Rules of the one-kernel PCG solve (k_pcg_team) that need no device code.
+#pragma once
+
+namespace idp {
+
+// Looks of the batched hand-over: both PCG loops look at the solves of a call
+// after 8, 24, 56, 120, 248, 504, 760, ... iterations of it (the two-kernel
+// loop's chunks of 8, 16, ... 256).  At the first look b by which half of the
+// solves have stopped, the others get as many iterations again and are handed
+// over after 2 b.
+constexpr int HAND_FIRST = 8;
+constexpr int HAND_LOOKS = 48;  // looks that a launch keeps count of: the last is at 11,256 iterations
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline int hand_next(int b)
+{
+    return b < 504 ? 2 * b + 8 : b + 256;
+}
+
+}  // namespace idp

@@ -129,3 +129,53 @@ def test_profiles_record_the_solve_that_runs():
             assert np.array_equal(runs[level][0], runs[1][0]) and np.array_equal(runs[level][1], runs[1][1])
     finally:
         d.close()
+
+
+def _served(scs, level, max_newton):
+    """The scenes started together in one engine: (engine calls, finishing
+    order with the call of each, states)."""
+    b = driver.BatchAnimFix(scs)
+    c = b.ctx
+    try:
+        c.profile(level)
+        c.serve_configure(b.h, pcg_rtol=b.pcg_rtol, max_newton=max_newton)
+        ids = list(range(len(scs)))
+        c.serve_start(ids, [s.X for s in scs], [s.velocity for s in scs], b.tol[ids], b.dHat2[ids], b.kappa[ids])
+        calls, order, left = 0, [], 1
+        while left:
+            left, fin = c.serve_iterate()
+            calls += 1
+            order += [(calls, int(i)) for i in np.nonzero(fin)[0]]
+        return calls, order, [c.serve_result(i)[:2] for i in ids]
+    finally:
+        b.close()
+
+
+def _rest(*cells):
+    X, tets = scenes.kuhn_block(*cells, 0.05)
+    return scenes.Scene("rest", X, tets, X.copy())
+
+
+# solves that stop at once beside a long one; solves that stop at different
+# looks; more instances, most of them long
+HANDOVER = [
+    ("stop_at_once", lambda: [_rest(2, 1, 1), _rest(3, 2, 2), scenes.bar_bend(20, 4, 4, 0.05, 0.15, 30.0)], 6),
+    ("mix", lambda: [scenes.small_bend(), scenes.cube_sinusoid(4, seed=3), scenes.cube_sinusoid(5, seed=7),
+                     scenes.bar_bend(20, 4, 4, 0.05, 0.15, 60.0)], 6),
+    ("uneven", lambda: [_rest(1, 1, 1)] + [scenes.cube_sinusoid(n, seed=n) for n in (2, 3, 9, 4, 12, 5, 7)], 5),
+]
+
+
+@pytest.mark.parametrize("name,make,newton", HANDOVER, ids=[h[0] for h in HANDOVER])
+def test_handover_points_are_those_of_the_two_kernels(name, make, newton):
+    """When solves are handed over decides how many engine calls a batch takes
+    and in which order frames finish: both equal the two-kernel loop's, and
+    the results are the same bits."""
+    scs = make()
+    want = _served(scs, 3, newton)
+    say(f"[pcg team] {name}: {want[0]} engine calls, finished {want[1]}")
+    for _ in range(2):
+        got = _served(scs, 0, newton)
+        assert got[:2] == want[:2], (got[:2], want[:2])
+        for (Xa, va), (Xb, vb) in zip(got[2], want[2]):
+            assert np.array_equal(Xa, Xb) and np.array_equal(va, vb)
