@@ -15,7 +15,6 @@
 #include "prim.hpp"
 #include "kernels.hpp"
 #include "linalg.hpp"
-#include "team_rule.hpp"
 
 namespace idp {
 
@@ -2234,6 +2233,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
         }
     if (nrun == 0) return false;
     if (coarse && L.coarse.K > 4 * (int)tab.size()) return false;
+    if (!one && !L.team_starts.now()) return false;
     TeamArgs T;
     T.tab = B == 1 ? nullptr : L.team_tab.upload_get(tab.data(), tab.size(), s);
     T.vbeg = I.d_vbeg.p;
@@ -2264,9 +2264,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     T.done = team + 1;
     T.start = (unsigned*)(team + 1 + B);
     T.hand = team + 1 + 2 * B;
-    // about 20 ms: other streams' kernels may hold CUs that long (IDP_TEAM_WAIT: another number of polls)
-    const char* wait = std::getenv("IDP_TEAM_WAIT");
-    T.start_limit = wait ? std::atol(wait) : 20000;
+    T.start_limit = L.team_wait;
     T.nstart = handover ? nrun : 0;
     T.spin_limit = 1L << 23;
     T.aptr = L.coarse.aptr.p;
@@ -2491,6 +2489,7 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
             run[i] = run[i] && hf[B + i] == 0 && hdone[i] == 0;  // its team did not start
             left |= run[i] != 0;
         }
+        L.team_starts.ended(!left);
         if (left) {
             teamed = false;
             tables();

@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "team_rule.hpp"
 
 namespace idp {
 
@@ -52,6 +53,8 @@ struct LinWork {
     DBuf<unsigned long long> team_words;
     unsigned long long team_tag = 0;  // last tag used in them
     int team_tok = -1;                // profiler token of the last one-kernel solve
+    long team_wait = TEAM_WAIT;       // polls of a team's start
+    TeamStarts team_starts;
     // cluster preconditioner
     DBuf<int> cl_best, cl_root, cl_size, cl_root2, cl_cnt, cl_mem, cl_cm4;
     DBuf<unsigned long long> cl_pack;

@@ -18,4 +18,26 @@ inline int hand_next(int b)
     return b < 504 ? 2 * b + 8 : b + 256;
 }
 
+// Starts of the one-kernel solves of a context.  A team whose workgroups do
+// not all become resident in time (other work holds compute units) leaves its
+// solve to the two-kernel loop after TEAM_WAIT polls, about a millisecond: as
+// long as a short solve takes.  While starts go on failing, the next 1, 3, 7,
+// ... 63 solves take that loop without a try, so a GPU that is busy for long
+// costs a context next to nothing; the results are the same either way.
+constexpr long TEAM_WAIT = 1000;
+struct TeamStarts {
+    int failed = 0, skip = 0;
+    bool now()
+    {
+        if (skip == 0) return true;
+        --skip;
+        return false;
+    }
+    void ended(bool started)
+    {
+        failed = started ? 0 : failed < 6 ? failed + 1 : 6;
+        skip = (1 << failed) - 1;
+    }
+};
+
 }  // namespace idp

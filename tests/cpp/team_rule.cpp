@@ -1,0 +1,62 @@
+// Host checks of the one-kernel PCG solve's rules (idp_amd/csrc/team_rule.hpp).
+#include <cstdio>
+#include <cstdlib>
+
+#include "../../idp_amd/csrc/team_rule.hpp"
+
+#define CHECK(c)                                                         \
+    do {                                                                 \
+        if (!(c)) {                                                      \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);          \
+            std::exit(1);                                                \
+        }                                                                \
+    } while (0)
+
+using namespace idp;
+
+// the looks are the two-kernel loop's chunk ends
+static void looks()
+{
+    int b = 0, chunk = 8, look = HAND_FIRST;
+    for (int k = 0; k < HAND_LOOKS; ++k) {
+        b += chunk;
+        chunk = 2 * chunk < 256 ? 2 * chunk : 256;
+        CHECK(look == b);
+        look = hand_next(look);
+    }
+    CHECK(b >= 10000);  // the default iteration limit of a step's solves
+}
+
+// while starts fail, tries get rare; one that succeeds brings every solve back
+static void starts()
+{
+    TeamStarts s;
+    for (int i = 0; i < 5; ++i) {
+        CHECK(s.now());
+        s.ended(true);
+    }
+    int tries = 0;
+    for (int i = 0; i < 1000; ++i)
+        if (s.now()) {
+            ++tries;
+            s.ended(false);
+        }
+    CHECK(tries <= 25);  // 6 on the way to one in 64, then one in 64
+    CHECK(tries >= 15);
+    while (!s.now()) {
+    }
+    s.ended(true);
+    for (int i = 0; i < 5; ++i) {
+        CHECK(s.now());
+        s.ended(true);
+    }
+    CHECK(TEAM_WAIT <= 2000);  // polls of about a microsecond: no longer than a short solve
+}
+
+int main()
+{
+    looks();
+    starts();
+    std::puts("ok");
+    return 0;
+}

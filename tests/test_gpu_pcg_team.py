@@ -2,6 +2,8 @@
 the two-kernel loop, so a Newton direction is the same bit for bit whichever
 runs it.  A batch of more rows than one launch holds takes the two-kernel
 loop."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -178,4 +180,42 @@ def test_handover_points_are_those_of_the_two_kernels(name, make, newton):
         got = _served(scs, 0, newton)
         assert got[:2] == want[:2], (got[:2], want[:2])
         for (Xa, va), (Xb, vb) in zip(got[2], want[2]):
+            assert np.array_equal(Xa, Xb) and np.array_equal(va, vb)
+
+
+@pytest.mark.parametrize("contexts", [2, 3])
+def test_contexts_on_threads_at_once_equal_alone(contexts):
+    """Contexts whose teams do not fit the GPU together (253 and 147
+    workgroups) step at the same time on threads of their own: whichever solves
+    leave for the two-kernel loop, every context ends as it does alone."""
+    scs = [scenes.bar_twist_fold(*dims, 0.05, seed=3, fold_radius=0.35 * dims[1] / 16)
+           for dims in ((80, 20, 18), (64, 16, 16), (40, 9, 9))[:contexts]]
+
+    def steps(d, sc, kappa, out):
+        for _ in range(2):
+            d.kappa[:] = kappa
+            d.ctx.set_state(sc.X)
+            d.set_target(sc.target)
+            d.advance_one_time_step(max_newton=6)
+            out.append(d.state())
+
+    def run(together):
+        ds = [driver.TetAnimFix(sc) for sc in scs]
+        outs = [[] for _ in scs]
+        th = [threading.Thread(target=steps, args=(d, sc, d.kappa.copy(), o)) for d, sc, o in zip(ds, scs, outs)]
+        for t in th:
+            t.start()
+            if not together:
+                t.join()
+        for t in th:
+            t.join()
+        for d in ds:
+            d.close()
+        return outs
+
+    say(f"[pcg team] {contexts} contexts at once")
+    alone, both = run(False), run(True)
+    for a, b in zip(alone, both):
+        assert len(a) == len(b) == 2
+        for (Xa, va), (Xb, vb) in zip(a, b):
             assert np.array_equal(Xa, Xb) and np.array_equal(va, vb)
