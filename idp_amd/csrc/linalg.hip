@@ -1231,8 +1231,6 @@ __global__ void __launch_bounds__(PCG_UPD_BLOCK * PCG_UPD_WAVES_MAX) k_pcg_updat
 // ---------------------------------------------------------------------------
 constexpr int TEAM_THREADS = 512;  // 2 wavefronts per SIMD: 256 registers a lane, room for the first rows' blocks
 constexpr int TEAM_WAVES = TEAM_THREADS / 64;
-constexpr int TEAM_MAX = 256;      // workgroups of a launch at most: one per CU
-constexpr int TEAM_ROWS = 128;     // rows of a workgroup: two per 8 lanes in the SpMV, 4 lanes a row in the update
 constexpr int TEAM_TASKS = 512;    // coarse aggregates at most (and, fewer, wavefront row sums)
 constexpr int TEAM_VALUES = 1952;  // values of one meeting at most (r_c of 320 aggregates)
 
@@ -2205,6 +2203,20 @@ __global__ void k_pcg_start(int B, const unsigned char* __restrict__ solve, int*
     err[i] = 0;
 }
 
+// workgroups of k_pcg_team that the context's device holds at once
+int team_resident()
+{
+    int dev = 0, cus = 0, per = INT_MAX;
+    IDP_HIP(hipGetDevice(&dev));
+    IDP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    for (const void* fn : {(const void*)k_pcg_team<false, false>, (const void*)k_pcg_team<false, true>}) {
+        int n = 0;
+        IDP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, TEAM_THREADS, 0));
+        per = std::min(per, n);
+    }
+    return per * cus;
+}
+
 // Runs the solves of the instances in `run` with k_pcg_team; false where the
 // two-kernel loop is used instead:
 //  - more rows than TEAM_MAX workgroups hold (32,768).  With the rest of the
@@ -2232,6 +2244,8 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
             one = one && t == 1;
         }
     if (nrun == 0) return false;
+    if (L.team_resident < 0) L.team_resident = team_resident();
+    if (!team_fits((int)tab.size(), one, L.team_resident)) return false;
     if (coarse && L.coarse.K > 4 * (int)tab.size()) return false;
     if (!one && !L.team_starts.now()) return false;
     TeamArgs T;

@@ -53,6 +53,7 @@ struct LinWork {
     DBuf<unsigned long long> team_words;
     unsigned long long team_tag = 0;  // last tag used in them
     int team_tok = -1;                // profiler token of the last one-kernel solve
+    int team_resident = -1;           // workgroups of one that the device holds at once (-1: not asked yet)
     long team_wait = TEAM_WAIT;       // polls of a team's start
     TeamStarts team_starts;
     // cluster preconditioner

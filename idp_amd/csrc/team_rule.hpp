@@ -3,6 +3,18 @@
 
 namespace idp {
 
+constexpr int TEAM_MAX = 256;   // workgroups of a launch at most: one per CU of the whole chip
+constexpr int TEAM_ROWS = 128;  // rows of a workgroup: two per 8 lanes in the SpMV, 4 lanes a row in the update
+
+// Workgroups that can run together: a team of several waits for all of its
+// members, so a launch with such a team has to fit the compute units that the
+// device shows (a partition of the chip shows fewer than 256); teams of one
+// wait for nobody.
+inline bool team_fits(int workgroups, bool all_of_one, int resident)
+{
+    return workgroups <= TEAM_MAX && (all_of_one || workgroups <= resident);
+}
+
 // Looks of the batched hand-over: both PCG loops look at the solves of a call
 // after 8, 24, 56, 120, 248, 504, 760, ... iterations of it (the two-kernel
 // loop's chunks of 8, 16, ... 256).  At the first look b by which half of the

@@ -53,8 +53,18 @@ static void starts()
     CHECK(TEAM_WAIT <= 2000);  // polls of about a microsecond: no longer than a short solve
 }
 
+// a launch needs all of its waiting workgroups resident at once
+static void fits()
+{
+    CHECK(team_fits(256, false, 256) && !team_fits(257, false, 512) && !team_fits(257, true, 256));
+    // a partition of 32 compute units
+    CHECK(team_fits(32, false, 32) && !team_fits(33, false, 32) && team_fits(33, true, 32));
+    CHECK(!team_fits(1, false, 0) && team_fits(1, true, 0));
+}
+
 int main()
 {
+    fits();
     looks();
     starts();
     std::puts("ok");
