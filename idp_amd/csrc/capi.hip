@@ -1465,8 +1465,9 @@ int idp_ctx_create(int device, idp_ctx** out)
             const int k = std::atoi(e);
             if (k >= 0 && k < 8) c->L.spmv_shape = k;
         }
-        // polls of a one-kernel solve's start (tests)
+        // polls of a one-kernel solve's start and of its waits (tests)
         if (const char* e = std::getenv("IDP_TEAM_WAIT")) c->L.team_wait = std::atol(e);
+        if (const char* e = std::getenv("IDP_TEAM_SPIN")) c->L.team_spin = std::atol(e);
     } catch (const HipError& e) {
         delete c->eng;
         delete c;

@@ -2280,7 +2280,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     T.hand = team + 1 + 2 * B;
     T.start_limit = L.team_wait;
     T.nstart = handover ? nrun : 0;
-    T.spin_limit = 1L << 23;
+    T.spin_limit = L.team_spin;
     T.aptr = L.coarse.aptr.p;
     T.avert = L.coarse.avert.p;
     T.Ps = L.coarse.Ps.p;
@@ -2305,7 +2305,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
 // -2 (breakdown, p.q <= 0); relres[i] = |r|/|b|.
 void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* b, double* x, double rtol,
                      int maxit, const unsigned char* solve_h, int* iters, double* relres, const unsigned char* warm,
-                     bool handover)
+                     bool handover, bool one_kernel)
 {
     const InstDev& I = m.inst;
     const int B = I.B;
@@ -2486,14 +2486,22 @@ void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* 
     int nstart = 0;
     for (int i = 0; i < B; ++i) nstart += run[i];
     std::vector<int> hdone(B, 0), tstop(B, -1);  // one-kernel solves: handed over / stopped after these iterations
-    bool teamed = nA > 0 && !(P && P->two_kernels()) && !A.red && shape.g == 8 &&
+    bool teamed = one_kernel && nA > 0 && !(P && P->two_kernels()) && !A.red && shape.g == 8 &&
                   pcg_team(L, s, I, A, run, team, coarse, handover && nstart > 1);
     if (teamed) {
         double* h = L.pin->as<double>(nres + (nints + 1) / 2);
         IDP_HIP(hipMemcpyAsync(h, scal, (nres + (nints + 1) / 2) * sizeof(double), hipMemcpyDeviceToHost, s));
         IDP_HIP(hipStreamSynchronize(s));
         const int* hi = (const int*)(h + nres);
-        if (hi[2 * B + 2]) throw HipError(IDP_E_HIP, "PCG: a workgroup's wait for its team ran out");
+        if (hi[2 * B + 2]) {
+            // a workgroup's wait for its team ran out: x and the vectors may be
+            // half written, so every solve starts again, from zero
+            if (P) P->end(IDP_K_PCG, tok);
+            L.team_starts.ended(false);
+            for (unsigned char& k : sv) k = k != 0;
+            pcg_solve_batch(L, s, m, b, x, rtol, maxit, sv.data(), iters, relres, nullptr, handover, false);
+            return;
+        }
         std::copy(h, h + 3 * B, hs.begin());
         std::copy(hi, hi + 2 * B, hf.begin());
         bool left = false;

@@ -56,6 +56,7 @@ struct LinWork {
     int team_resident = -1;           // workgroups of one that the device holds at once (-1: not asked yet)
     long team_wait = TEAM_WAIT;       // polls of a team's start
     TeamStarts team_starts;
+    long team_spin = 1L << 23;        // polls of a started team's waits (some seconds)
     // cluster preconditioner
     DBuf<int> cl_best, cl_root, cl_size, cl_root2, cl_cnt, cl_mem, cl_cm4;
     DBuf<unsigned long long> cl_pack;
@@ -90,10 +91,11 @@ void init_erow(LinWork& L, hipStream_t s, const MeshDev& m, const std::vector<in
 // (their previous direction) instead of zero.  handover: once half of the
 // solves have stopped, the rest get as many iterations again and are then
 // handed over (iters = PCG_HANDED_OVER); a hand-over changes no arithmetic.
+// one_kernel false: the two-kernel loop whatever the size.
 constexpr int PCG_HANDED_OVER = -3;
 void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* b, double* x, double rtol,
                      int maxit, const unsigned char* solve_h, int* iters, double* relres,
-                     const unsigned char* warm = nullptr, bool handover = false);
+                     const unsigned char* warm = nullptr, bool handover = false, bool one_kernel = true);
 int pcg_solve_persistent(LinWork& L, hipStream_t s, const MeshDev& m, const double* b, double* x, double rtol,
                          int maxit, double* relres, const unsigned char* warm = nullptr);
 double dev_dot(LinWork& L, hipStream_t s, long n, const double* a, const double* b);

@@ -219,3 +219,37 @@ def test_contexts_on_threads_at_once_equal_alone(contexts):
         assert len(a) == len(b) == 2
         for (Xa, va), (Xb, vb) in zip(a, b):
             assert np.array_equal(Xa, Xb) and np.array_equal(va, vb)
+
+
+def test_a_team_whose_wait_runs_out_starts_the_solve_again(monkeypatch):
+    """With one poll per wait a started team gives up at a meet: the call does
+    not fail, its solves run again in the two-kernel loop.  A direction starts
+    from zero either way, so it is the same bits; a step loses its warm starts
+    and ends where the oracle's tolerance says (1e-6 of the diagonal)."""
+    def run(make):
+        b = make()
+        try:
+            if isinstance(b, driver.TetAnimFix):
+                return [_direction(b, b.scene, 2, cv) for cv in (-1, 48)]
+            b.advance_one_time_step()
+            return [b.state(i)[0] for i in range(len(b.scenes))]
+        finally:
+            b.close()
+
+    def bar():
+        return driver.TetAnimFix(_scene(33, 9, 7))
+
+    batch = [scenes.small_bend(), scenes.cube_sinusoid(5, seed=7), scenes.small_bend(angle_deg=200.0)]
+
+    def mix():
+        return driver.BatchAnimFix(batch)
+
+    want = [run(bar), run(mix)]
+    monkeypatch.setenv("IDP_TEAM_SPIN", "1")
+    say("[pcg team] one poll per wait")
+    got = [run(bar), run(mix)]
+    for (g0, s0, i0, _, upd0), (g1, s1, i1, _, upd1) in zip(want[0], got[0]):
+        assert upd0 == 0 and upd1 > 0  # the one kernel without the limit, the two kernels with it
+        assert i0 == i1 and np.array_equal(g0, g1) and np.array_equal(s0, s1)
+    for sc, X0, X1 in zip(batch, want[1], got[1]):
+        assert np.abs(X0 - X1).max() <= 1e-6 * sc.diag
