@@ -2231,7 +2231,8 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
               bool coarse, bool handover)
 {
     const int B = I.B;
-    std::vector<int4> tab;
+    std::vector<int4>& tab = L.h_team_tab;  // kept: its upload may be under way when this returns
+    tab.clear();
     bool one = true;
     int nrun = 0;
     for (int i = 0; i < B; ++i)
@@ -2249,16 +2250,16 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     if (coarse && L.coarse.K > 4 * (int)tab.size()) return false;
     if (!one && !L.team_starts.now()) return false;
     TeamArgs T;
-    T.tab = B == 1 ? nullptr : L.team_tab.upload_get(tab.data(), tab.size(), s);
-    T.vbeg = I.d_vbeg.p;
-    T.it0 = nullptr;
-    for (int i = 0; i < B; ++i)
-        if (run[i] && L.h_it0[i]) T.it0 = L.team_it0.upload_get(L.h_it0.data(), B, s);
     T.K = coarse ? L.coarse.K : 0;
     T.ncd = L.coarse.ncd;
     T.nfree = L.coarse.nfree;
     T.lda = L.coarse.lda;
     if (T.K && (T.ncd > TEAM_VALUES || T.K > TEAM_TASKS)) return false;
+    T.tab = B == 1 ? nullptr : L.team_tab.upload_get(tab.data(), tab.size(), s);
+    T.vbeg = I.d_vbeg.p;
+    bool cont = false;
+    for (int i = 0; i < B; ++i) cont |= run[i] && L.h_it0[i];
+    T.it0 = cont ? L.team_it0.upload_get(L.h_it0.data(), B, s) : nullptr;
     // published words; tags only grow, so words of earlier launches never match (cleared when they would wrap)
     const size_t n_pq = 2 * (size_t)A.nbA, n_r = 2 * (2 * (size_t)A.nbB + 8 * B), n_c = 2 * 7 * (size_t)T.K;
     const size_t nw = n_pq + n_r + n_c;

@@ -50,6 +50,7 @@ struct LinWork {
     DBuf<double> pinv, r, z, p, p1, q, part0, part1, part2, part3, part_bx, scal, scal2, red;
     DBuf<int> team_it0;  // one-kernel solve: iterations of earlier calls
     DBuf<int4> team_tab;
+    std::vector<int4> h_team_tab;
     DBuf<unsigned long long> team_words;
     unsigned long long team_tag = 0;  // last tag used in them
     int team_tok = -1;                // profiler token of the last one-kernel solve
