@@ -2244,7 +2244,7 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
             for (int k = 0; k < t; ++k) tab.push_back(make_int4(i, k, t, 0));
             one = one && t == 1;
         }
-    if (nrun == 0) return false;
+    if (nrun == 0 || !team_addresses(A.nV)) return false;
     if (L.team_resident < 0) L.team_resident = team_resident();
     if (!team_fits((int)tab.size(), one, L.team_resident)) return false;
     if (coarse && L.coarse.K > 4 * (int)tab.size()) return false;

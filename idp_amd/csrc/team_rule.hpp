@@ -15,6 +15,12 @@ inline bool team_fits(int workgroups, bool all_of_one, int resident)
     return workgroups <= TEAM_MAX && (all_of_one || workgroups <= resident);
 }
 
+// The kernel's vectors are buffers with 32-bit byte offsets over the whole
+// context, the two copies of p (48 bytes a vertex) the longest of them: a
+// batch of more than 89 million vertices, however few of its solves run, is
+// out of their range.
+inline bool team_addresses(long long nV) { return 48 * nV <= 0xffffffffll; }
+
 // Looks of the batched hand-over: both PCG loops look at the solves of a call
 // after 8, 24, 56, 120, 248, 504, 760, ... iterations of it (the two-kernel
 // loop's chunks of 8, 16, ... 256).  At the first look b by which half of the

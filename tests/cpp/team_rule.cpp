@@ -62,9 +62,18 @@ static void fits()
     CHECK(!team_fits(1, false, 0) && team_fits(1, true, 0));
 }
 
+// every byte offset of the longest vector fits 32 bits
+static void addresses()
+{
+    CHECK(team_addresses(32768) && team_addresses(89478485));
+    CHECK(48ll * 89478485 <= 0xffffffffll && 48ll * 89478486 > 0xffffffffll);
+    CHECK(!team_addresses(89478486) && !team_addresses(0x7fffffff));
+}
+
 int main()
 {
     fits();
+    addresses();
     looks();
     starts();
     std::puts("ok");
