@@ -1414,8 +1414,12 @@ __device__ inline double wave_sum_dpp(double x)
     return x;
 }
 
-// r.z of update block b in the second meeting's values (r.r two further): the
-// two blocks of a chunk fill a 64-byte line, which one workgroup writes
+// r.z of update block b in the second meeting's values (r.r two further): two
+// blocks fill a 64-byte line, a workgroup's own where their number is even.
+// Where it is odd most workgroups write halves of two lines (a split that
+// gives each its line and the last one the single block was no faster: one
+// direction of the 43x11x9 bar 1.33 ms either way, the bent 20x4x4 bar 0.5%
+// slower)
 __device__ inline int team_rblk(int b) { return 4 * (b >> 1) + (b & 1); }
 struct TeamRblk {
     __device__ int operator()(int b) const { return team_rblk(b); }
@@ -1643,8 +1647,11 @@ __device__ inline double team_row(const PcgArgs& A, const TeamBuf& bz, const Tea
     return wave_sum_dpp(d);
 }
 
-// COARSE: with the coarse level (T.K > 0)
-template <bool ONE, bool COARSE>
+// COARSE: with the coarse level (T.K > 0); HAND: solves may be handed over
+// (T.nstart > 0, never with the coarse level).  Variants of their own, since
+// the registers are full: the hand-over's few values cost the twisted 64x16x16
+// bar 1.6% of its step in spills.
+template <bool ONE, bool COARSE, bool HAND>
 __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T)
 {
     __shared__ double wt[TEAM_TASKS];
@@ -1685,10 +1692,14 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
     double* sci = A.scal + 3 * inst;
     double rz = 0.0, rr = 0.0, rzo = 1.0, bb = 0.0;
     int hand = 0;
-    // the next look of this solve (k-th) and the next look whose answer it needs
-    int look = HAND_FIRST, klook = 0, ans = HAND_FIRST, kans = 0;
-    const bool counts = T.nstart && rank == 0 && tid == 0;
-    if (counts) atomicAdd(T.hand + 2 * HAND_LOOKS, 1);
+    // hand-over, by one thread of the solve: its next look (and which), the next look whose answer it needs
+    __shared__ int look[2], ans[2];
+    const bool counts = HAND && rank == 0 && tid == 0;
+    if (counts) {
+        look[0] = ans[0] = HAND_FIRST;
+        look[1] = ans[1] = 0;
+        atomicAdd(T.hand + 2 * HAND_LOOKS, 1);
+    }
     if (tid == 0) bad = 0;
     // ---- the workgroup's blocks and update state stay in registers
     const int gl = lane & 7;
@@ -1774,14 +1785,14 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
         const unsigned tag = T.tag0 + 1u + (unsigned)(it - it_first);
         const int par = it & 1;
         // the same decisions in every workgroup of the team
-        if (hand) {
+        if (HAND && hand) {
             state = -1;
             break;
         }
-        if (it - it_first == look) {
-            if (counts && klook < HAND_LOOKS) atomicAdd(T.hand + klook, 1);
-            look = hand_next(look);
-            ++klook;
+        if (counts && it - it_first == look[0]) {
+            if (look[1] < HAND_LOOKS) atomicAdd(T.hand + look[1], 1);
+            look[0] = hand_next(look[0]);
+            ++look[1];
         }
         if (!(bb > 0.0) || (it > 0 && rr <= A.rtol2 * bb)) {
             state = 1;
@@ -1884,21 +1895,24 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
         // an odd number of blocks: the last line's other half is published too, so that all of it is waited for
         if (wave == 1 && lane < 2 && (nb & 1) && rank == size - 1)
             team_put<ONE>(w_r, nr, val, team_rblk(nb) + 2 * lane, 0.0, tag);
-        const bool asks = it + 1 - it_first == 2 * ans;
-        if (counts) team_put<ONE>(w_r, nr, val, nr - 1, asks && team_hand(T, kans) ? 1.0 : 0.0, tag);
-        if (asks) {
-            ans = hand_next(ans);
-            ++kans;
+        if (counts) {
+            double mark = 0.0;
+            if (it + 1 - it_first == 2 * ans[0]) {
+                if (team_hand(T, ans[1])) mark = 1.0;
+                ans[0] = hand_next(ans[0]);
+                ++ans[1];
+            }
+            team_put<ONE>(w_r, nr, val, nr - 1, mark, tag);
         }
-        if (!team_meet<ONE>(T, w_r, T.nstart ? nr : nr - 1, tag, val, &bad)) return;
+        if (!team_meet<ONE>(T, w_r, HAND ? nr : nr - 1, tag, val, &bad)) return;
         if (wave == 0) {
             const double s = team_sum(val, nb, TeamRblk());
             if (lane == 0) sh[0] = s;
         } else if (wave == 1) {
             const double s = team_sum(val + 2, nb, TeamRblk());
             if (lane == 0) sh[1] = s;
-        } else if (wave == 2 && lane == 0) {
-            sh[5] = T.nstart ? val[nr - 1] : 0.0;
+        } else if (HAND && wave == 2 && lane == 0) {
+            sh[5] = val[nr - 1];
         }
         if (COARSE) {
             __syncthreads();  // val is read above and written by the next meeting
@@ -1994,7 +2008,7 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
         __syncthreads();
         rz = sh[0];
         rr = sh[1];
-        hand = sh[5] != 0.0;
+        if (HAND) hand = sh[5] != 0.0;
         if (COARSE) rz += sh[2];
     }
     // ---- the solve stopped or is handed over
@@ -2010,7 +2024,7 @@ __global__ void __launch_bounds__(TEAM_THREADS) k_pcg_team(PcgArgs A, TeamArgs T
     A.flag[inst] = state;
     if (state != 2) sci[1] = rr;
     sci[2] = (double)it;
-    if (counts && klook < HAND_LOOKS) atomicAdd(T.hand + HAND_LOOKS + klook, 1);  // stopped before its next look
+    if (counts && look[1] < HAND_LOOKS) atomicAdd(T.hand + HAND_LOOKS + look[1], 1);  // stopped before its next look
 }
 
 // generic deterministic sum of partials -> out[0]
@@ -2209,7 +2223,8 @@ int team_resident()
     int dev = 0, cus = 0, per = INT_MAX;
     IDP_HIP(hipGetDevice(&dev));
     IDP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    for (const void* fn : {(const void*)k_pcg_team<false, false>, (const void*)k_pcg_team<false, true>}) {
+    for (const void* fn : {(const void*)k_pcg_team<false, false, false>, (const void*)k_pcg_team<false, true, false>,
+                           (const void*)k_pcg_team<false, false, true>}) {
         int n = 0;
         IDP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, TEAM_THREADS, 0));
         per = std::min(per, n);
@@ -2286,9 +2301,11 @@ bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, con
     T.avert = L.coarse.avert.p;
     T.Ps = L.coarse.Ps.p;
     T.Ainv = L.coarse.Ainv.p;
-    static const void* const fns[] = {(const void*)k_pcg_team<false, false>, (const void*)k_pcg_team<false, true>,
-                                      (const void*)k_pcg_team<true, false>, (const void*)k_pcg_team<true, true>};
-    const void* fn = fns[(one ? 2 : 0) + (coarse ? 1 : 0)];
+    static const void* const fns[] = {
+        (const void*)k_pcg_team<false, false, false>, (const void*)k_pcg_team<false, true, false>,
+        (const void*)k_pcg_team<false, false, true>,  (const void*)k_pcg_team<true, false, false>,
+        (const void*)k_pcg_team<true, true, false>,   (const void*)k_pcg_team<true, false, true>};
+    const void* fn = fns[(one ? 3 : 0) + (coarse ? 1 : handover ? 2 : 0)];
     PcgArgs a = A;
     void* args[] = {&a, &T};
     hipEvent_t e0 = nullptr, e1 = nullptr;

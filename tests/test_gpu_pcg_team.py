@@ -230,7 +230,7 @@ def test_a_team_whose_wait_runs_out_starts_the_solve_again(monkeypatch):
         b = make()
         try:
             if isinstance(b, driver.TetAnimFix):
-                return [_direction(b, b.scene, 2, cv) for cv in (-1, 48)]
+                return [_direction(b, b.scene, 2, cv) for cv in (-1, 144)]
             b.advance_one_time_step()
             return [b.state(i)[0] for i in range(len(b.scenes))]
         finally:
