@@ -1342,13 +1342,15 @@ __device__ inline bool team_meet(const TeamArgs& T, const unsigned long long* w,
 // but only one process can hold that queue), so a workgroup that has waited
 // too long for the others leaves, if the team is still incomplete, and then
 // all of them do: the solve was not touched and runs in the two-kernel loop.
+// (A limit of 0 starts the teams whose workgroups come together, a negative
+// one none.)
 constexpr unsigned TEAM_LEFT = 0x80000000u;
 __device__ inline bool team_start(unsigned* word, unsigned size, long limit)
 {
     unsigned w = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
     for (long k = 0;; ++k) {
         if (w & TEAM_LEFT) return false;
-        if (w == size) return true;
+        if (w == size && limit >= 0) return true;
         if (k >= limit && __hip_atomic_compare_exchange_strong(word, &w, w | TEAM_LEFT, __ATOMIC_RELAXED,
                                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             return false;  // (on failure w is the word as it stands)

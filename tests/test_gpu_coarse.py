@@ -77,3 +77,45 @@ def test_coarse_level_is_deterministic_and_bounded_on_a_large_mesh():
         assert rel0 <= 1e-8
     finally:
         d.close()
+
+
+# orders of A_c of 48 (one tile of 64 rows), 108 and 162 (two and three tiles,
+# both with a ragged end), 384 (six whole tiles), 750 and 1728
+@pytest.mark.parametrize("cells", [(1, 1, 1), (2, 2, 1), (2, 2, 2), (3, 3, 3), (4, 4, 4), (5, 5, 7)])
+def test_coarse_inverse_is_exact_when_the_coarse_space_is_everything(cells):
+    """With one vertex per aggregate the coarse space holds every vector, so
+    z = (Z + A^-1) r and the preconditioned operator is Z A + I.  Every tet
+    touches at most four clusters, so the eigenvalues of Z A lie in (0, 4] and
+    those of Z A + I in (1, 5]: CG's error falls by 2 rho^k, rho = (sqrt 5 - 1)
+    / (sqrt 5 + 1), and the residual by that times sqrt(cond A).  An inverse
+    that is not A's breaks the bound; the cluster preconditioner by itself is
+    far from it on these systems (a step of 1 s: stiffness over mass)."""
+    X, tets = scenes.kuhn_block(*cells, 0.05)
+    rng = np.random.default_rng(3)
+    X = X + rng.normal(0.0, 5e-4, X.shape)
+    sc = scenes.Scene("block", X, tets, X + rng.normal(0.0, 1e-2, X.shape), h=1.0)
+    d = driver.TetAnimFix(sc)
+    try:
+        def direction(cv):
+            return d.ctx.newton_direction(sc.X, sc.target, sc.h, d.dHat2, d.kappa[0], pcg_rtol=1e-10, coarse_verts=cv)
+
+        _, s0, _, it0 = direction(-1)
+        g, s1, rel, it1 = direction(1)
+        rp, col, val = d.ctx.get_bsr()
+        n = len(rp) - 1
+        A = np.zeros((n, 3, n, 3))
+        for r in range(n):
+            for k in range(rp[r], rp[r + 1]):
+                A[r, :, col[k], :] += val[k]
+        A = A.reshape(3 * n, 3 * n)
+        ev = np.linalg.eigvalsh(0.5 * (A + A.T))
+        rho = (np.sqrt(5) - 1) / (np.sqrt(5) + 1)
+        most = int(np.ceil(np.log(2 * np.sqrt(ev[-1] / ev[0]) / 1e-10) / -np.log(rho)))
+        say(f"[coarse] {n} vertices, condition {ev[-1] / ev[0]:.1e}: {it0} iterations without, {it1} with, at most {most}")
+        assert rel <= 1e-10 and it1 <= most
+        if n >= 27:
+            assert it0 > 1.5 * most
+        # |A s + g| <= 1e-10 |g| up to the residual's own rounding
+        assert np.linalg.norm(A @ s1 + g) <= 2e-10 * np.linalg.norm(g) + 1e-15 * ev[-1] * np.linalg.norm(s1) * n
+    finally:
+        d.close()

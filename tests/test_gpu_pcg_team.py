@@ -1,7 +1,8 @@
 """The PCG solve as one kernel on MI355X: its sums are formed in the order of
 the two-kernel loop, so a Newton direction is the same bit for bit whichever
 runs it.  A batch of more rows than one launch holds takes the two-kernel
-loop."""
+loop, and so does any solve at profile level 3.  Which of the two ran is read
+from a profile: one SpMV record and no update record for the one kernel."""
 import threading
 
 import numpy as np
@@ -24,6 +25,18 @@ def _scene(nx, ny, nz, seed=5):
     return scenes.Scene(f"bar{nx}x{ny}x{nz}", X, tets, scenes.sinusoid_target(X, side, 4, (0.2, 0.4), (0.5, 1.0), rng))
 
 
+def _direction(d, sc, level, coarse=-1, X=None):
+    """One Newton direction at a profile level; (gradient, direction, PCG
+    iterations, one-kernel solves, launches of the update kernel seen)."""
+    d.ctx.profile(level)
+    g, s, r, it = d.ctx.newton_direction(sc.X if X is None else X, sc.target, sc.h, d.dHat2, d.kappa[0],
+                                         pcg_rtol=1e-10, coarse_verts=coarse)
+    p = d.ctx.profile_read()
+    d.ctx.profile(0)
+    assert r <= 1e-10
+    return g, s, it, p["pcg_spmv"]["launches"], p["pcg_update"]["launches"]
+
+
 # rows of the first instance: 8 (less than a wavefront's), 64 and 66 (one
 # 64-row block, one and two rows more), 126 and 130 (one workgroup and the
 # next), 195 (odd number of 64-row blocks, two workgroups)
@@ -34,8 +47,12 @@ def test_one_kernel_equals_two_kernels(cells):
     a, b = driver.BatchAnimFix([sc]), driver.BatchAnimFix([sc, big])
     try:
         say(f"[pcg team] {sc.X.shape[0]} rows alone, then beside {big.X.shape[0]}")
-        a.advance_one_time_step(max_newton=2)
-        b.advance_one_time_step(max_newton=2)
+        for d in (a, b):
+            d.ctx.profile(2)
+            d.advance_one_time_step(max_newton=2)
+        pa, pb = a.ctx.profile_read(), b.ctx.profile_read()
+        assert pa["pcg_spmv"]["launches"] == 2 and pa["pcg_update"]["launches"] == 0
+        assert pb["pcg_update"]["launches"] > 0
         Xa, va = a.state(0)
         Xb, vb = b.state(0)
         assert np.array_equal(Xa, Xb) and np.array_equal(va, vb)
@@ -44,24 +61,76 @@ def test_one_kernel_equals_two_kernels(cells):
         b.close()
 
 
-@pytest.mark.parametrize("cells,verts", [((20, 4, 4), 48), ((33, 9, 7), 144), ((64, 16, 16), 144), ((40, 40, 1), 64)])
+# 5, 22, 147 and 27 workgroups; 5, 48, 208 and 25 aggregates (the second more
+# than two per workgroup, the last a sheet, whose thin direction is one voxel)
+@pytest.mark.parametrize("cells,verts", [((20, 4, 4), 144), ((33, 9, 7), 100), ((64, 16, 16), 144), ((40, 40, 1), 144)])
 def test_one_kernel_with_coarse_level(cells, verts):
     """The direction agrees with the one without a coarse level to the solves'
-    residual, and a second solve of the same system gives the same bits."""
+    residual, a second solve of the same system gives the same bits, and so do
+    the kernels of the two-kernel loop."""
     sc = _scene(*cells)
     d = driver.TetAnimFix(sc)
     try:
-        def direction(cv):
-            return d.ctx.newton_direction(sc.X, sc.target, sc.h, d.dHat2, d.kappa[0], pcg_rtol=1e-10, coarse_verts=cv)
-
-        g0, s0, r0, i0 = direction(-1)
-        g1, s1, r1, i1 = direction(verts)
-        g2, s2, r2, i2 = direction(verts)
+        g0, s0, i0, n0, u0 = _direction(d, sc, 2)
+        g1, s1, i1, n1, u1 = _direction(d, sc, 2, verts)
+        g2, s2, i2, _, _ = _direction(d, sc, 2, verts)
+        g3, s3, i3, _, u3 = _direction(d, sc, 3, verts)
         say(f"[pcg team] {sc.X.shape[0]} rows: {i0} iterations without the coarse level, {i1} with it")
-        assert r0 <= 1e-10 and r1 <= 1e-10
+        assert (n0, u0) == (n1, u1) == (1, 0) and u3 > 0
         assert np.array_equal(g0, g1) and np.array_equal(s1, s2) and i1 == i2
+        assert np.array_equal(g1, g3) and np.array_equal(s1, s3) and i1 == i3
         # |error| <= cond |residual|: 1e-8 holds for systems of condition below 100
         assert np.linalg.norm(s1 - s0) <= 1e-8 * np.linalg.norm(s0)
+    finally:
+        d.close()
+
+
+def _plates(nx, nz, n, gap, seed=4):
+    """n plates of nx x 1 x nz cells, facing surfaces gap times the contact
+    distance apart and shifted by a fraction of a cell, pressed together."""
+    P, T = scenes.kuhn_block(nx, 1, nz, 0.05)
+    rng = np.random.default_rng(seed)
+    g = gap * 1e-3 * 0.05 * np.sqrt((nx + 1) ** 2 + n ** 2 + (nz + 1) ** 2)
+    X = np.vstack([P + [rng.uniform(0.01, 0.04), k * (0.05 + g), rng.uniform(0.01, 0.04)] for k in range(n)])
+    X[:, [0, 2]] += rng.normal(0.0, 1e-3, (X.shape[0], 2))
+    X[:, 1] += rng.uniform(-0.1, 0.1, X.shape[0]) * g
+    tets = np.vstack([T + k * P.shape[0] for k in range(n)]).astype(np.int32)
+    return scenes.Scene("plates", X, tets, X * [1.0, 0.9, 1.0])
+
+
+def _hub_ball(level):
+    """A ball of one tet per triangle of an icosphere, all around its centre
+    (vertex 0): one row coupled with every vertex."""
+    X, tris = scenes.icosphere(level, 0.5)
+    X = np.vstack([[0.0, 0.0, 0.0], X])
+    rng = np.random.default_rng(2)
+    X = X + rng.normal(0.0, 1e-4, X.shape)
+    tets = np.hstack([np.zeros((tris.shape[0], 1), np.int32), tris + 1]).astype(np.int32)
+    return scenes.Scene("ball", X, tets, X * [1.1, 0.95, 1.0])
+
+
+@pytest.mark.parametrize("coarse", [-1, 144])
+@pytest.mark.parametrize("make", [lambda: _plates(24, 21, 3, 0.5), lambda: _plates(30, 30, 2, 0.4),
+                                  lambda: _hub_ball(3), lambda: _hub_ball(4)],
+                         ids=["plates24x21x3", "plates30x30x2", "ball642", "ball2562"])
+def test_long_rows_and_many_columns_equal_two_kernels(make, coarse):
+    """Rows of more than the 16 blocks that a workgroup keeps in registers
+    (contact; the centre of a ball) and workgroups of more than the 1,024
+    columns that it stages."""
+    sc = make()
+    d = driver.TetAnimFix(sc)
+    try:
+        g0, s0, i0, n0, u0 = _direction(d, sc, 2, coarse)
+        g1, s1, i1, _, u1 = _direction(d, sc, 3, coarse)
+        rp, col, _ = d.ctx.get_bsr()
+        longest = int(np.diff(rp).max())
+        columns = max(np.unique(col[rp[a]:rp[min(a + 128, len(rp) - 1)]]).size for a in range(0, len(rp) - 1, 128))
+        say(f"[pcg team] {sc.name}, {sc.X.shape[0]} rows: longest {longest} blocks, {columns} columns of 128 rows")
+        assert longest > (16 if "plates" in sc.name else 512)
+        if sc.X.shape[0] == 2563:
+            assert columns > 1024
+        assert (n0, u0) == (1, 0) and u1 > 0
+        assert i0 == i1 and np.array_equal(g0, g1) and np.array_equal(s0, s1)
     finally:
         d.close()
 
@@ -84,35 +153,24 @@ def test_batch_of_many_small_meshes_in_one_kernel():
 
 
 def test_a_team_that_does_not_start_leaves_the_solve_to_the_two_kernels(monkeypatch):
-    """With no patience for workgroups that are not resident yet, the first
-    workgroup leaves and the solve runs in the two-kernel loop: same bits."""
+    """With no patience at all (a negative number of polls) the workgroups leave
+    and the solve runs in the two-kernel loop: same bits."""
     sc = _scene(20, 4, 4)
 
     def solve(cv):
         d = driver.TetAnimFix(sc)
-        r = d.ctx.newton_direction(sc.X, sc.target, sc.h, d.dHat2, d.kappa[0], coarse_verts=cv)
+        r = _direction(d, sc, 2, cv)
         d.close()
         return r
 
-    for cv in (-1, 48):
-        g0, s0, _, i0 = solve(cv)
-        monkeypatch.setenv("IDP_TEAM_WAIT", "0")
+    for cv in (-1, 144):
+        g0, s0, i0, _, u0 = solve(cv)
+        monkeypatch.setenv("IDP_TEAM_WAIT", "-1")
         say(f"[pcg team] coarse {cv}: no wait for the team")
-        g1, s1, _, i1 = solve(cv)
+        g1, s1, i1, _, u1 = solve(cv)
         monkeypatch.delenv("IDP_TEAM_WAIT")
+        assert u0 == 0 and u1 > 0
         assert i0 == i1 and np.array_equal(g0, g1) and np.array_equal(s0, s1)
-
-
-def _direction(d, sc, level, coarse=-1, X=None):
-    """One Newton direction at a profile level; (gradient, direction, PCG
-    iterations, one-kernel solves, launches of the update kernel seen)."""
-    d.ctx.profile(level)
-    g, s, r, it = d.ctx.newton_direction(sc.X if X is None else X, sc.target, sc.h, d.dHat2, d.kappa[0],
-                                         pcg_rtol=1e-10, coarse_verts=coarse)
-    p = d.ctx.profile_read()
-    d.ctx.profile(0)
-    assert r <= 1e-10
-    return g, s, it, p["pcg_spmv"]["launches"], p["pcg_update"]["launches"]
 
 
 def test_profiles_record_the_solve_that_runs():
