@@ -156,19 +156,30 @@ __global__ void k_coarse_diag(int n, double* __restrict__ Ac)
 // ---- inverse of A_c by blocked symmetric sweeps --------------------------
 // Sweeping block k of a symmetric matrix: B_kk = -A_kk^-1, B_ik = A_ik A_kk^-1,
 // B_ij = A_ij - A_ik A_kk^-1 A_kj; after all blocks B = -A^-1, symmetric
-// throughout, so only the lower tiles are formed.  One launch per block of
-// SW rows, one workgroup per lower tile, reading one copy of the matrix and
-// writing the other; the workgroup of the next diagonal tile also inverts it,
-// so a launch is the whole serial step.  (A library Cholesky and inverse took
-// 2.2 ms of small dependent kernels at order 780 and 5 ms at 1,900.)
+// throughout, so only the lower tiles are formed.  A_kk^-1 = T^T T enters by
+// T = L^-1 of the tile's Cholesky factor, B_ij = A_ij - U_i^T U_j with
+// U_j = T A_kj: what is left of the matrix is then the Cholesky one, with its
+// error (a stiff contact gives A_c a condition of 1e12; with A_kk^-1 itself
+// the error was 1,000 times a Cholesky inverse's there, pivots went negative
+// and the level was refused).  One launch per block of SW rows, one workgroup
+// per lower tile, reading one copy of the matrix and writing the other; the
+// workgroup of the next diagonal tile also factors it, so a launch is the whole
+// serial step.  (A library Cholesky and inverse took 2.2 ms of small dependent
+// kernels at order 780 and 5 ms at 1,900.)
 constexpr int SW = 64;
 constexpr int SW_LD = SW + 1;
 
-// M (SW x SW, symmetric positive definite, in LDS) -> its inverse, by scalar
-// sweeps; each thread keeps a 4 x 4 piece, the pivot row goes through row
-// (2 x SW).  *ok: every pivot was positive.
-__device__ inline void sweep_invert(double (*M)[SW_LD], double* row, int* ok)
+// M (SW x SW, symmetric positive definite, in LDS) -> T = L^-1, M = L L^T.
+// Row operations that eliminate below each pivot, with the unit lower factor's
+// inverse growing in place of the eliminated columns, then each row by the root
+// of its pivot.  Each thread keeps a 4 x 4 piece; four pivot rows at a time go
+// through rows, and every thread brings its columns of them up to date by
+// itself (with a barrier per pivot the 24 sweeps of order 1,536 took 8 us more
+// each; 51 us now, as with A_kk^-1 in T's place).
+// *ok: every pivot was positive.
+__device__ inline void sweep_factor(double (*M)[SW_LD], double (*rows)[4][SW], int* ok)
 {
+#pragma clang fp contract(fast)
     const int ti = (threadIdx.x >> 4) * 4, tj = (threadIdx.x & 15) * 4;
     double a[4][4];
 #pragma unroll
@@ -176,38 +187,69 @@ __device__ inline void sweep_invert(double (*M)[SW_LD], double* row, int* ok)
 #pragma unroll
         for (int j = 0; j < 4; ++j) a[i][j] = M[ti + i][tj + j];
     bool good = true;
-#pragma unroll 4
-    for (int p = 0; p < SW; ++p) {
-        double* r = row + SW * (p & 1);
-        const int pi = p & 3;
-        if (ti == (p & ~3)) {
+    for (int p = 0; p < SW; p += 4) {
+        double(*r)[SW] = rows[(p >> 2) & 1];
+        if (ti == p) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) r[tj + j] = pi == 0 ? a[0][j] : pi == 1 ? a[1][j] : pi == 2 ? a[2][j] : a[3][j];
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) r[i][tj + j] = a[i][j];
         }
         __syncthreads();
-        const double d = r[p];
-        good = good && d > 0;
-        const double id = 1.0 / d;
-        double ri[4], rj[4];
+        double P[4][4], R[4][4], F[4][4];  // the pivot rows in the pivot, this thread's and (below: by symmetry) its rows' columns
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            ri[i] = r[ti + i];
-            rj[i] = r[tj + i];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const bool oi = ti + i == p, oj = tj + j == p;
-                const double s = ri[i] * id;
-                a[i][j] = oi ? (oj ? -id : rj[j] * id) : (oj ? s : a[i][j] - s * rj[j]);
+                P[q][j] = r[q][p + j];
+                R[q][j] = r[q][tj + j];
+                F[q][j] = r[q][ti + j];
             }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const double d = P[q][q];
+            good = good && d > 0;
+            const double id = 1.0 / d;
+            // the block's later pivot rows
+#pragma unroll
+            for (int b = q + 1; b < 4; ++b) {
+                const double f = P[q][b] * id;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j > q) P[b][j] = P[b][j] - f * P[q][j];
+                    R[b][j] = tj + j == p + q ? -f : R[b][j] - f * R[q][j];
+                    F[b][j] = F[b][j] - f * F[q][j];
+                }
+            }
+            // this thread's rows below the block
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double f = F[q][i] * id;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const double t = tj + j == p + q ? -f : a[i][j] - f * R[q][j];
+                    a[i][j] = ti > p ? t : a[i][j];
+                }
+            }
+        }
+        if (ti == p)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) a[i][j] = R[i][j];
     }
     __syncthreads();
+    double* piv = rows[0][0];
+    if (ti == tj)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) piv[ti + i] = a[i][i];  // the pivots
+    __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 4; ++j) M[ti + i][tj + j] = -a[i][j];
+    for (int i = 0; i < 4; ++i) {
+        const double s = 1.0 / sqrt(piv[ti + i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) M[ti + i][tj + j] = tj + j < ti + i ? a[i][j] * s : tj + j == ti + i ? s : 0.0;
+    }
     if (!good && threadIdx.x == 0) *ok = 0;
     __syncthreads();
 }
@@ -223,8 +265,19 @@ __device__ inline void sweep_load(const double* __restrict__ A, int n, int i, in
     }
 }
 
-// C (4 x 4 per thread) = X Y, both SW x SW in LDS
-__device__ inline void sweep_mul(const double (*X)[SW_LD], const double (*Y)[SW_LD], double (*c)[4])
+__device__ inline void sweep_put(const double (*c)[4], double (*T)[SW_LD])
+{
+    const int ti = (threadIdx.x >> 4) * 4, tj = (threadIdx.x & 15) * 4;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) T[ti + u][tj + v] = c[u][v];
+}
+
+// C (4 x 4 per thread) = X Y, or X^T Y (TX), both SW x SW in LDS, over the
+// inner indices [k0, k1): the rest is zero where X is the lower triangle T
+template <bool TX>
+__device__ inline void sweep_mul(const double (*X)[SW_LD], const double (*Y)[SW_LD], int k0, int k1, double (*c)[4])
 {
 #pragma clang fp contract(fast)
     const int ti = (threadIdx.x >> 4) * 4, tj = (threadIdx.x & 15) * 4;
@@ -233,11 +286,11 @@ __device__ inline void sweep_mul(const double (*X)[SW_LD], const double (*Y)[SW_
 #pragma unroll
         for (int j = 0; j < 4; ++j) c[i][j] = 0.0;
 #pragma unroll 4
-    for (int k = 0; k < SW; ++k) {
+    for (int k = k0; k < k1; ++k) {
         double x[4], y[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            x[u] = X[ti + u][k];
+            x[u] = TX ? X[k][ti + u] : X[ti + u][k];
             y[u] = Y[k][tj + u];
         }
 #pragma unroll
@@ -247,27 +300,27 @@ __device__ inline void sweep_mul(const double (*X)[SW_LD], const double (*Y)[SW_
     }
 }
 
-// inverse of the first diagonal tile
+// T of the first diagonal tile
 __global__ void __launch_bounds__(256) k_coarse_first(int n, const double* __restrict__ A, double* __restrict__ D,
                                                       int* __restrict__ info)
 {
-    __shared__ double M[SW][SW_LD], row[2 * SW];
+    __shared__ double M[SW][SW_LD], rows[2][4][SW];
     __shared__ int ok;
     if (threadIdx.x == 0) ok = 1;
     sweep_load(A, n, 0, 0, M);
     __syncthreads();
-    sweep_invert(M, row, &ok);
+    sweep_factor(M, rows, &ok);
     for (int e = threadIdx.x; e < SW * SW; e += 256) D[e] = M[e / SW][e % SW];
     if (threadIdx.x == 0) *info = ok ? 0 : 1;
 }
 
-// sweep of block k: src -> dst; D = A_kk^-1, Dn receives the next one.  The
-// last sweep (k = n / SW - 1) writes the inverse itself, both triangles.
+// sweep of block k: src -> dst; D = T of the block, Dn receives the next one.
+// The last sweep (k = n / SW - 1) writes the inverse itself, both triangles.
 __global__ void __launch_bounds__(256) k_coarse_sweep(int n, int k, const double* __restrict__ src,
                                                       double* __restrict__ dst, const double* __restrict__ D,
                                                       double* __restrict__ Dn, int* __restrict__ info)
 {
-    __shared__ double X[SW][SW_LD], Y[SW][SW_LD], row[2 * SW];
+    __shared__ double X[SW][SW_LD], Y[SW][SW_LD], rows[2][4][SW];
     __shared__ int ok;
     const int nt = n / SW;
     int i = (int)((sqrt(8.0 * blockIdx.x + 1.0) - 1.0) / 2.0);
@@ -275,33 +328,43 @@ __global__ void __launch_bounds__(256) k_coarse_sweep(int n, int k, const double
     while (i * (i + 1) / 2 > (int)blockIdx.x) --i;
     const int j = (int)blockIdx.x - i * (i + 1) / 2;  // lower tile (i, j)
     const int ti = (threadIdx.x >> 4) * 4, tj = (threadIdx.x & 15) * 4;
+    const int r0 = 16 * (threadIdx.x >> 6), r1 = r0 + 16;  // the wavefront's rows: T is zero right of, T^T left of them
     const bool last = k == nt - 1;
     const double sg = last ? -1.0 : 1.0;
     if (threadIdx.x == 0) ok = 1;
     for (int e = threadIdx.x; e < SW * SW; e += 256) X[e / SW][e % SW] = D[e];
     double c[4][4];
-    bool trans = false;  // c holds the transpose of the tile
+    const bool trans = j == k && i != k;  // c holds the transpose of the tile
     if (i == k && j == k) {
         __syncthreads();
+        sweep_mul<true>(X, X, r0, SW, c);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) c[u][v] = -X[ti + u][tj + v];
+            for (int v = 0; v < 4; ++v) c[u][v] = -c[u][v];
     } else {
-        // W = D A_kj (tile row k), or for j == k: D A_ki, the transpose of A_ik D
-        trans = j == k;
         sweep_load(src, n, k, trans ? i : j, Y);
         __syncthreads();
-        sweep_mul(X, Y, c);
-        if (i != k && j != k) {
+        sweep_mul<false>(X, Y, 0, r1, c);  // U of the tile's column (row, for j == k)
+        if (i == k || j == k) {
             __syncthreads();
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) Y[ti + u][tj + v] = c[u][v];
-            sweep_load(src, n, i, k, X);
+            sweep_put(c, Y);
             __syncthreads();
-            sweep_mul(X, Y, c);
+            sweep_mul<true>(X, Y, r0, SW, c);  // A_kk^-1 A_kj
+        } else {
+            double u[4][4];
+            if (i != j) {
+                __syncthreads();
+                sweep_load(src, n, k, i, Y);
+                __syncthreads();
+                sweep_mul<false>(X, Y, 0, r1, u);
+            }
+            __syncthreads();
+            sweep_put(c, Y);
+            if (i != j) sweep_put(u, X);
+            else sweep_put(c, X);
+            __syncthreads();
+            sweep_mul<true>(X, Y, 0, SW, c);
             __syncthreads();
             sweep_load(src, n, i, j, X);
             __syncthreads();
@@ -330,7 +393,7 @@ __global__ void __launch_bounds__(256) k_coarse_sweep(int n, int k, const double
         for (int y = y0; y < SW; y += 4) dst[(size_t)(SW * i + y) * n + SW * j + x] = sg * X[y][x];
     if (i == k + 1 && j == k + 1) {
         __syncthreads();
-        sweep_invert(X, row, &ok);
+        sweep_factor(X, rows, &ok);
         for (int e = threadIdx.x; e < SW * SW; e += 256) Dn[e] = X[e / SW][e % SW];
         if (threadIdx.x == 0 && !ok) *info = 1;
     }
