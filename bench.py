@@ -53,12 +53,12 @@ def workload(name):
     raise SystemExit(f"unknown workload {name}")
 
 
-def read_traffic(path, kernel):
-    """HBM bytes per dispatch of `kernel` from a committed counter summary
-    (a line "traffic_bytes_per_dispatch <kernel>: <bytes>"), or None."""
+def read_traffic(path, kernel, per="dispatch"):
+    """HBM bytes per dispatch (or PCG iteration) of `kernel` from a committed
+    counter summary (a line "traffic_bytes_per_<per> <kernel>: <bytes>"), or None."""
     if not os.path.exists(path):
         return None
-    m = re.search(r"traffic_bytes_per_dispatch\s+" + re.escape(kernel) + r":\s*([0-9.eE+]+)", open(path).read())
+    m = re.search(rf"traffic_bytes_per_{per}\s+" + re.escape(kernel) + r":\s*([0-9.eE+]+)", open(path).read())
     return float(m.group(1)) if m else None
 
 
@@ -616,7 +616,8 @@ def bench_plain(a):
         extra["roofline_update_kernel"] = _roofline("pcg_update", prof_t, a.traffic)
     elif roof:
         roof["kernel"] = "pcg_team"
-        roof["traffic"] = None
+        t = read_traffic(a.traffic, "pcg_team", "iteration")
+        roof["traffic"] = t and t * sum(state["pcg"]) / max(roof["launches_sampled"], 1)
     state["extra"] = extra
 
     # per-family device times: a profiled solve truncated to a bounded number

@@ -8,9 +8,10 @@
 // over precomputed per-block contribution lists; C holds the contact blocks
 // of the current constraint set, built by radix-sorting (row,col) keys of all
 // local blocks and reducing each run in sort order.  Every sum has a fixed
-// order, so results are bitwise reproducible.  PCG uses the 3x3 block-Jacobi
-// preconditioner; its dot products are deterministic two-level reductions
-// whose final sum is recomputed by each consumer block.
+// order, so results are bitwise reproducible.  PCG is preconditioned by block
+// Jacobi over clusters of up to four vertices, for one mesh with a coarse level
+// (coarse.hip); its dot products are deterministic two-level reductions whose
+// final sum is recomputed by each consumer block.
 #include "common.hpp"
 #include "prim.hpp"
 #include "kernels.hpp"
@@ -2240,8 +2241,11 @@ int team_resident()
 //    rows read from memory an iteration of 24 cubes (41,580 rows) took 18 us,
 //    against 15 us in the two kernels;
 //  - a coarse level of more than two aggregates per workgroup and 256-thread
-//    half: a thin sheet of 625 free vertices (10 workgroups) has 320 of them,
-//    and took 1.2 ms more per solve than the four kernels.
+//    half (a sheet of 625 free vertices cut into 320 aggregates, 32 for each of
+//    its 10 workgroups, took 1.2 ms more per solve than the four kernels);
+//  - launches whose teams the device cannot hold together, contexts of more
+//    vertices than 32-bit offsets reach, and, for a while, contexts whose teams
+//    found the device taken (team_rule.hpp).
 // Below, per iteration and with launch gaps: 81 rows 24 -> 5 us, 18,785 rows
 // with 100-130 aggregates 40 -> 30-39 us.
 bool pcg_team(LinWork& L, hipStream_t s, const InstDev& I, const PcgArgs& A, const std::vector<char>& run, int* team,

@@ -89,9 +89,10 @@ void init_erow(LinWork& L, hipStream_t s, const MeshDev& m, const std::vector<in
 // solve_h (host, B; null = all new): 0 not solving, 1 new solve, 2 continue
 // a solve handed over by the previous call.  warm (device, B bytes; null =
 // none): new solves that start from a multiple of what x holds on entry
-// (their previous direction) instead of zero.  handover: once half of the
-// solves have stopped, the rest get as many iterations again and are then
-// handed over (iters = PCG_HANDED_OVER); a hand-over changes no arithmetic.
+// (their previous direction) instead of zero.  handover: at the first look
+// (team_rule.hpp) by which half of the solves have stopped, the rest get as
+// many iterations again and are then handed over (iters = PCG_HANDED_OVER); a
+// hand-over changes no arithmetic.
 // one_kernel false: the two-kernel loop whatever the size.
 constexpr int PCG_HANDED_OVER = -3;
 void pcg_solve_batch(LinWork& L, hipStream_t s, const MeshDev& m, const double* b, double* x, double rtol,

@@ -6,11 +6,12 @@
 
 `solve` runs the first Newton iterations of the 64x16x16 twist-and-fold bar
 (one mesh, the default solver options).  `analyze` groups the trace's
-consecutive PCG kernels (SpMV, update, their partial-sum reductions and the coarse level) into
-runs, one run per chunk of enqueued iterations, and reports the kernels'
-device time against the runs' span: the difference is the time between
-kernels inside a run, which is what capturing the chunk in a graph could
-remove at most.  Prints one JSON object.
+consecutive PCG kernels into runs and reports the kernels' device time against
+the runs' span: the difference is the time between kernels inside a run, which
+is what capturing it in a graph could remove at most.  A run is one solve of
+up to 32,768 rows (k_pcg_team), or a chunk of enqueued iterations of a larger
+one (SpMV, update, their partial-sum reductions and the coarse level).  Prints
+one JSON object.
 """
 from __future__ import annotations
 

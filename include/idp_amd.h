@@ -51,8 +51,10 @@ typedef struct idp_solver_opts {
                            default (65536), < 0: never.  Results do not depend on it. */
     int pcg_handover;   /* batched engine: 0 (default): once half of the instances' PCG solves have
                            stopped, the others run as many iterations again and then continue in the
-                           next Newton iteration while the rest go on; < 0: never.  Results do not
-                           depend on it. */
+                           next Newton iteration while the rest go on; < 0: never.  Looked for after
+                           8, 24, 56, ... iterations, so the engine calls of a batch are the same
+                           from run to run, unless other work on the GPU keeps solves from starting
+                           together.  Results do not depend on it. */
     int accd_max_steps; /* additive-CCD steps one pair may take in one step-size call before it is
                            taken as a hit at the time of impact it reached (a smaller, still
                            conservative step).  0: the default, IDP_ACCD_MAX_STEPS_DEFAULT; < 0: no

@@ -21,6 +21,8 @@ def test_committed_traffic_summary_is_read_for_the_roofline():
     path = os.path.join(ROOT, "profiles", "k_pcg_spmv_traffic_bar_twist_fold.txt")
     t = bench.read_traffic(path, "pcg_spmv")
     assert t is not None and 2e7 < t < 4e7  # bytes per SpMV dispatch on the 64x16x16 bar
+    t = bench.read_traffic(path, "pcg_team", "iteration")
+    assert t is not None and 1e7 < t < 2.7e7  # per iteration of the one-kernel solve: below one pass over matrix and vectors
     assert bench.read_traffic(path, "no_such_kernel") is None
     assert bench.read_traffic(os.path.join(ROOT, "profiles", "absent.txt"), "pcg_spmv") is None
 
